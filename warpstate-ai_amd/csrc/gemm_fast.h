@@ -56,10 +56,12 @@ constexpr int kFNT = kFWM * kFWN * kWave;               // 512 threads
 constexpr int kFTileBytes = 256 * kFBK * 2;             // one operand tile, 32 KiB
 constexpr int kFStageBytes = 2 * kFTileBytes;
 constexpr int kFLdsBytes = 2 * kFStageBytes;            // 128 KiB
-// Epilogue staging: each wave's 64 x 128 BF16 tile, rows padded to 272 bytes so that both
-// the fragment-order writes and the row-order 16-byte reads are bank-conflict free.
-constexpr int kFStageRow = 272;
-constexpr int kFStageWave = 64 * kFStageRow;
+// Epilogue staging: each wave's BF16 tile of FA x FB blocks (64 x 128 here), rows padded by
+// 16 bytes (to 272) so that both the fragment-order writes and the row-order 16-byte reads
+// are bank-conflict free.
+template <int FB> constexpr int epi_row() { return FB * 32 + 16; }
+template <int FA, int FB> constexpr int epi_wave() { return FA * 16 * epi_row<FB>(); }
+constexpr int kFStageWave = epi_wave<4, 8>();
 constexpr int kFLdsAlloc = 8 * kFStageWave > kFLdsBytes ? 8 * kFStageWave : kFLdsBytes;
 // Both operands K-contiguous: A in two stages, B in three (the whole 160 KiB of a CU).
 constexpr int kFLdsAllocKK = 5 * kFTileBytes;
@@ -245,7 +247,9 @@ struct FEpiStore {
   __device__ __forceinline__ static void run(const GemmParams& p, Acc16<FA, FB>& acc, int m_base,
                                              int n_base, int lane, int tm, int tn, int wn,
                                              unsigned char* stage) {
-    static_assert(FA * 16 == 64 && FB * 16 == 128, "staging holds a 64 x 128 wave tile");
+    // LPR lanes cover a row of the wave tile (8 columns each), RPI rows per instruction.
+    constexpr int kRow = epi_row<FB>(), LPR = FB * 2, RPI = 64 / LPR, NQ = FA * 16 / RPI;
+    static_assert(64 % LPR == 0 && NQ >= 1, "whole rows per instruction");
     opaque_lane(lane);
     // Fragment order -> staging rows, sigmoid applied, every value rounded to BF16. The
     // gate test is made once per wave for its 128 columns (n_base is wave-uniform): with a
@@ -265,7 +269,7 @@ struct FEpiStore {
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = f(acc.v[i][j][e], n_base + c + e);
           u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-          *reinterpret_cast<u32x2_t*>(stage + r * kFStageRow + c * 2) = w;
+          *reinterpret_cast<u32x2_t*>(stage + r * kRow + c * 2) = w;
         }
     };
     if (gate == kNone) {
@@ -281,17 +285,17 @@ struct FEpiStore {
     // The accumulators are dead from here; the loads below must not be hoisted above.
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's staging writes landed
-    // Row order: lane (16 per row) owns 8 columns; 4 rows per instruction.
-    const int c8 = 8 * (lane & 15);
+    // Row order: lane (LPR per row) owns 8 columns.
+    const int c8 = 8 * (lane % LPR);
     const int n = n_base + c8;
     const bool full = n + 7 < p.N, half = n + 3 < p.N;  // N % 4 == 0 (vec_out)
     __amdgpu_buffer_rsrc_t rc = make_rsrc(p.c + (long)m_base * p.ldc + n_base, 0x7fffffff);
-    u32x4_t rv[16];
+    u32x4_t rv[NQ];
     if (RESIDUAL) {
       __amdgpu_buffer_rsrc_t rr = make_rsrc(p.aux + (long)m_base * p.ldaux + n_base, 0x7fffffff);
 #pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int r = 4 * q + (lane >> 4);
+      for (int q = 0; q < NQ; ++q) {
+        const int r = RPI * q + lane / LPR;
         const bool ok = m_base + r < p.M;
         const long off = (long)r * p.ldaux + c8;
         if (full) {
@@ -304,10 +308,10 @@ struct FEpiStore {
       }
     }
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int r = 4 * q + (lane >> 4);
+    for (int q = 0; q < NQ; ++q) {
+      const int r = RPI * q + lane / LPR;
       const bool ok = m_base + r < p.M;
-      u32x4_t vd = *reinterpret_cast<const u32x4_t*>(stage + r * kFStageRow + c8 * 2);
+      u32x4_t vd = *reinterpret_cast<const u32x4_t*>(stage + r * kRow + c8 * 2);
       if (RESIDUAL) {
 #pragma unroll
         for (int d = 0; d < 4; ++d)
@@ -334,7 +338,9 @@ struct FEpiSwiglu {
   __device__ __forceinline__ static void run(const GemmParams& p, Acc16<FA, FB>& acc, int m_base,
                                              int n_base, int lane, int tm, int tn, int wn,
                                              unsigned char* stage) {
-    static_assert(FA * 16 == 64 && FB * 16 == 128, "staging holds a 64 x 128 wave tile");
+    // FB / 2 blocks are up columns; LPR lanes cover one half's columns of a row.
+    constexpr int kRow = epi_row<FB>(), LPR = FB, RPI = 64 / LPR, NQ = FA * 16 / RPI;
+    static_assert(64 % LPR == 0 && NQ >= 1, "whole rows per instruction");
     opaque_lane(lane);
 #pragma unroll
     for (int i = 0; i < FA; ++i)
@@ -343,11 +349,11 @@ struct FEpiSwiglu {
         const int r = 16 * i + (lane & 15), c = 16 * j + 4 * (lane >> 4);
         u32x2_t w = {pack_bf16x2(acc.v[i][j][0], acc.v[i][j][1]),
                      pack_bf16x2(acc.v[i][j][2], acc.v[i][j][3])};
-        *reinterpret_cast<u32x2_t*>(stage + r * kFStageRow + c * 2) = w;
+        *reinterpret_cast<u32x2_t*>(stage + r * kRow + c * 2) = w;
       }
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's staging writes landed
-    const int c8 = 8 * (lane & 7);
+    const int c8 = 8 * (lane % LPR);
     const int n = n_base + c8;  // column in [0, H)
     const bool full = n + 7 < p.H, half = n + 3 < p.H;  // H % 4 == 0 (vec_out)
     __amdgpu_buffer_rsrc_t rp = make_rsrc(p.c + (long)m_base * p.ldc + n_base, 0x7fffffff);
@@ -355,11 +361,11 @@ struct FEpiSwiglu {
     const long hoff = p.H;
     const bool eager = p.eager;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int r = 8 * q + (lane >> 3);
+    for (int q = 0; q < NQ; ++q) {
+      const int r = RPI * q + lane / LPR;
       const bool ok = m_base + r < p.M;
-      const u32x4_t vu = *reinterpret_cast<const u32x4_t*>(stage + r * kFStageRow + c8 * 2);
-      const u32x4_t vg = *reinterpret_cast<const u32x4_t*>(stage + r * kFStageRow + (64 + c8) * 2);
+      const u32x4_t vu = *reinterpret_cast<const u32x4_t*>(stage + r * kRow + c8 * 2);
+      const u32x4_t vg = *reinterpret_cast<const u32x4_t*>(stage + r * kRow + (8 * FB + c8) * 2);
       u32x4_t va;
       // The rounding mode is tested once per row group, not per element (the compiler
       // otherwise computes both and selects).
@@ -424,10 +430,12 @@ struct FEpiSwigluBwd {
   __device__ __forceinline__ static void run(const GemmParams& p, Acc16<FA, FB>& acc, int m_base,
                                              int n_base, int lane, int tm, int tn, int wn,
                                              unsigned char* stage) {
+    constexpr int kRow = epi_row<FB>(), LPR = FB * 2, RPI = 64 / LPR, NQ = FA * 16 / RPI;
+    static_assert(64 % LPR == 0 && NQ >= 1, "whole rows per instruction");
     opaque_lane(lane);
     const long hoff = p.H;
     {
-      // Fragment order -> staging rows (64 x 128 BF16, 272-byte rows).
+      // Fragment order -> staging rows (the wave tile in BF16, padded rows).
 #pragma unroll
       for (int i = 0; i < FA; ++i)
 #pragma unroll
@@ -435,55 +443,50 @@ struct FEpiSwigluBwd {
           const int r = 16 * i + (lane & 15), c = 16 * j + 4 * (lane >> 4);
           u32x2_t v = {pack_bf16x2(acc.v[i][j][0], acc.v[i][j][1]),
                        pack_bf16x2(acc.v[i][j][2], acc.v[i][j][3])};
-          *reinterpret_cast<u32x2_t*>(stage + r * kFStageRow + c * 2) = v;
+          *reinterpret_cast<u32x2_t*>(stage + r * kRow + c * 2) = v;
         }
       // Keep the scheduler from hoisting the loads below above the staging writes (the
       // accumulators must be dead before the loaded rows take their registers).
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's staging writes landed
-      const int c8 = 8 * (lane & 15);       // this lane's 8 columns
+      const int c8 = 8 * (lane % LPR);      // this lane's 8 columns
       const int n = n_base + c8;
       // Buffer bases at this wave's tile origin keep the byte offsets small.
       __amdgpu_buffer_rsrc_t rp = make_rsrc(p.aux + (long)m_base * p.ldaux + n_base, 0x7fffffff);
       __amdgpu_buffer_rsrc_t rd = make_rsrc(p.c + (long)m_base * p.ldc + n_base, 0x7fffffff);
-      // All 16 rows' saved up/gate values are requested first (128 VGPRs; the
-      // accumulators are dead once staged), so the four row groups below wait for one
-      // memory latency instead of four.
-      u32x4_t vu[4][4], vg[4][4];
+      // All rows' saved up/gate values are requested first (128 VGPRs for a 64 x 128
+      // wave tile; the accumulators are dead once staged), so the row groups below wait
+      // for one memory latency instead of one each.
+      u32x4_t vu[NQ], vg[NQ];
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const int r = 16 * q + 4 * h + (lane >> 4);
-          const int m = m_base + r;
-          const bool ok = m < p.M && n + 7 < p.N;
-          const long off = (long)r * p.ldaux + c8;
-          vu[q][h] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rp, store_off(ok, off, 2), 0, kEpiNT));
-          vg[q][h] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rp, store_off(ok, off + hoff, 2), 0, kEpiNT));
-        }
+      for (int q = 0; q < NQ; ++q) {
+        const int r = RPI * q + lane / LPR;
+        const int m = m_base + r;
+        const bool ok = m < p.M && n + 7 < p.N;
+        const long off = (long)r * p.ldaux + c8;
+        vu[q] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rp, store_off(ok, off, 2), 0, kEpiNT));
+        vg[q] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rp, store_off(ok, off + hoff, 2), 0, kEpiNT));
+      }
       // The rounding mode is tested once here, not per element (the compiler otherwise
       // computes both and selects).
       auto finish = [&](auto eager) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < NQ; ++q) {
+          const int r = RPI * q + lane / LPR;
+          const int m = m_base + r;
+          const bool ok = m < p.M && n + 7 < p.N;
+          const u32x4_t vd = *reinterpret_cast<const u32x4_t*>(stage + r * kRow + c8 * 2);
+          u32x4_t od, og;
 #pragma unroll
-          for (int h = 0; h < 4; ++h) {
-            const int r = 16 * q + 4 * h + (lane >> 4);
-            const int m = m_base + r;
-            const bool ok = m < p.M && n + 7 < p.N;
-            const u32x4_t vd = *reinterpret_cast<const u32x4_t*>(stage + r * kFStageRow + c8 * 2);
-            u32x4_t od, og;
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-              unsigned wu, wg;
-              math2<decltype(eager)::value>(vd[d], vu[q][h][d], vg[q][h][d], wu, wg);
-              od[d] = wu;
-              og[d] = wg;
-            }
-            const long off = (long)r * p.ldc + c8;
-            __builtin_amdgcn_raw_buffer_store_b128(od, rd, store_off(ok, off, 2), 0, kEpiNT);
-            __builtin_amdgcn_raw_buffer_store_b128(og, rd, store_off(ok, off + hoff, 2), 0, kEpiNT);
+          for (int d = 0; d < 4; ++d) {
+            unsigned wu, wg;
+            math2<decltype(eager)::value>(vd[d], vu[q][d], vg[q][d], wu, wg);
+            od[d] = wu;
+            og[d] = wg;
           }
+          const long off = (long)r * p.ldc + c8;
+          __builtin_amdgcn_raw_buffer_store_b128(od, rd, store_off(ok, off, 2), 0, kEpiNT);
+          __builtin_amdgcn_raw_buffer_store_b128(og, rd, store_off(ok, off + hoff, 2), 0, kEpiNT);
         }
       };
       if (p.eager) finish(std::true_type{});
@@ -509,8 +512,7 @@ struct FEpiAccF32 {
                                              Acc16<FA, FB>& acc, int m_base, int n_base, int lane,
                                              int tm, int tn) {
     opaque_lane(lane);
-    const int m0 = tm * kFBM, n0 = tn * kFBN;
-    __amdgpu_buffer_rsrc_t rg = make_rsrc(g + (long)m0 * ldg + n0, 0x7fffffff);
+    __amdgpu_buffer_rsrc_t rg = make_rsrc(g + (long)m_base * ldg + n_base, 0x7fffffff);
 #pragma unroll
     for (int i = 0; i < FA; ++i) {
       const int m = m_base + 16 * i + (lane & 15);
@@ -520,7 +522,7 @@ struct FEpiAccF32 {
         const int n = n_base + 16 * j + 4 * (lane >> 4);
         {
           const bool ok = mok && (n + 3 < N);
-          const unsigned off = store_off(ok, (long)(m - m0) * ldg + (n - n0), 4);
+          const unsigned off = store_off(ok, (long)(m - m_base) * ldg + (n - n_base), 4);
           f32x4_t add;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -649,7 +651,7 @@ struct FEpiCEGrad {
         const int r = 16 * i + (lane & 15), c = 16 * j + 4 * (lane >> 4);
         u32x2_t w = {pack_bf16x2(acc.v[i][j][0], acc.v[i][j][1]),
                      pack_bf16x2(acc.v[i][j][2], acc.v[i][j][3])};
-        *reinterpret_cast<u32x2_t*>(stage + r * kFStageRow + c * 2) = w;
+        *reinterpret_cast<u32x2_t*>(stage + r * epi_row<FB>() + c * 2) = w;
       }
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's staging writes landed
@@ -665,7 +667,7 @@ struct FEpiCEGrad {
       const long tgt = ok ? p.targets[m] : -100;
       const float lse = ok ? p.lse[m] : 0.0f;
       const float scale = (tgt == -100) ? 0.0f : *p.grad_scale;
-      const u32x4_t vl = *reinterpret_cast<const u32x4_t*>(stage + r * kFStageRow + c8 * 2);
+      const u32x4_t vl = *reinterpret_cast<const u32x4_t*>(stage + r * epi_row<FB>() + c8 * 2);
       u32x4_t o;
       // The one-hot term only where some lane of the wave holds its row's target among
       // its 8 columns (for 4 rows x 128 columns of a 32768 vocabulary, 1 in 64); elsewhere
@@ -712,7 +714,7 @@ struct FEpiCEStatsLogits {
         const int r = 16 * i + (lane & 15), c = 16 * j + 4 * (lane >> 4);
         u32x2_t w = {pack_bf16x2(acc.v[i][j][0], acc.v[i][j][1]),
                      pack_bf16x2(acc.v[i][j][2], acc.v[i][j][3])};
-        *reinterpret_cast<u32x2_t*>(stage + r * kFStageRow + c * 2) = w;
+        *reinterpret_cast<u32x2_t*>(stage + r * epi_row<FB>() + c * 2) = w;
       }
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's staging writes landed
@@ -724,7 +726,7 @@ struct FEpiCEStatsLogits {
     for (int q = 0; q < 16; ++q) {
       const int r = 4 * q + (lane >> 4);
       const bool ok = m_base + r < p.M;
-      const u32x4_t vl = *reinterpret_cast<const u32x4_t*>(stage + r * kFStageRow + c8 * 2);
+      const u32x4_t vl = *reinterpret_cast<const u32x4_t*>(stage + r * epi_row<FB>() + c8 * 2);
       const long off = (long)r * p.ldc + c8;
       if (full) {
         __builtin_amdgcn_raw_buffer_store_b128(vl, rc, store_off(ok, off, 2), 0, kEpiNT);

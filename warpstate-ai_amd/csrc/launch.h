@@ -4,7 +4,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
-#include "gemm_fast.h"
+#include "gemm_ring.h"
 
 namespace ws {
 
@@ -176,6 +176,124 @@ int dispatch_fast(const GemmParams& p, int am, int bm, LaunchCfg cfg, hipStream_
     case 2: return run_fast<kMNContig, kKContig, PAIRED, Epi>(p, cfg, s);
     default: return run_fast<kMNContig, kMNContig, PAIRED, Epi>(p, cfg, s);
   }
+}
+
+// Macro-tiles of the vector-operand GEMMs: 256 x 256 (gemm_fast.h) and the ring kernel's
+// smaller ones (gemm_ring.h). Two 64 to 80 KiB workgroups fit a CU except for kTile128x1,
+// which takes the CU alone with eight waves and four stages.
+typedef RingCfg<128, 128, 2, 2, 2> Ring128x2;
+typedef RingCfg<128, 128, 4, 2, 4> Ring128x1;
+typedef RingCfg<64, 128, 2, 2, 3> Ring64x128;
+typedef RingCfg<64, 64, 2, 2, 4> Ring64;
+enum FastTile { kTile256 = 0, kTile128x2, kTile128x1, kTile64x128, kTile64, kFastTiles };
+
+// Cost of one launch of each macro-tile in microseconds, from a sweep of 32 shapes (128 to
+// 16384 rows, 512 to 32768 columns, K 512 to 16384; outputs of all tiles the same bits):
+// a CU runs its workgroups one after another (or two at a time), each taking `alone` us per
+// 64-deep k-tile, `pair` us for two that share the CU, and `fixed` us around its k-loop.
+// The 256 x 256 tile costs less per product with every CU busy; below about one round of
+// its tiles most CUs idle, and a smaller tile wins although it loads its operands more
+// often. Measured, us (256 x 256 against the choice): 512 x 1280 x 8960 159 / 40 (64 x 64),
+// 1999 x 1280 x 8960 158 / 71 (128 x 128 alone), 4096 x 1280 x 6400 114 / 71 (128 x 128
+// paired), 128 x 4800 x 960 23 / 7.4 (64 x 64); and where it stays: 8192 x 10240 x 2048
+// 250 / 294, 8192 x 2048 x 2048 54 / 59 (the best smaller tile).
+struct TileCost {
+  int bm, bn;
+  float alone, pair, fixed;  // pair 0: one workgroup per CU
+};
+inline const TileCost& tile_cost(int tile, int am, int bm) {
+  static const TileCost kk[kFastTiles] = {{256, 256, 1.55f, 0.0f, 4.0f},
+                                          {128, 128, 0.62f, 0.93f, 3.2f},
+                                          {128, 128, 0.50f, 0.0f, 3.6f},
+                                          {64, 128, 0.34f, 0.55f, 3.6f},
+                                          {64, 64, 0.28f, 0.36f, 3.4f}};
+  static const TileCost kmn[kFastTiles] = {{256, 256, 1.87f, 0.0f, 4.0f},
+                                           {128, 128, 0.64f, 0.95f, 3.2f},
+                                           {128, 128, 0.53f, 0.0f, 3.6f},
+                                           {64, 128, 0.38f, 0.58f, 3.6f},
+                                           {64, 64, 0.31f, 0.38f, 3.4f}};
+  static const TileCost mnmn[kFastTiles] = {{256, 256, 1.85f, 0.0f, 4.0f},
+                                            {128, 128, 0.60f, 1.00f, 3.2f},
+                                            {128, 128, 0.54f, 0.0f, 3.6f},
+                                            {64, 128, 0.39f, 0.70f, 3.6f},
+                                            {64, 64, 0.29f, 0.42f, 3.4f}};
+  if (am == kKContig && bm == kKContig) return kk[tile];
+  return (am == kMNContig && bm == kMNContig ? mnmn : kmn)[tile];
+}
+// An [m, n] output (n the packed width of a paired GEMM) over k_tiles k-tiles.
+inline float tile_time(int tile, long m, long n, long k_tiles, int am, int bm, int cus) {
+  const TileCost& c = tile_cost(tile, am, bm);
+  const long tiles = (long)cdiv(m, c.bm) * cdiv(n, c.bn), rounds = tiles / cus;
+  const float kt = (float)k_tiles;
+  if (tile == kTile256) {
+    // With most CUs idle in the last round its tiles' loads meet less traffic.
+    float t = (float)rounds * (c.alone * kt + c.fixed);
+    if (tiles % cus) t += c.alone * (0.73f + 0.27f * (float)(tiles % cus) / (float)cus) * kt + c.fixed;
+    return t;
+  }
+  const long per_cu = rounds + (tiles % cus != 0);
+  if (c.pair == 0.0f) return (float)per_cu * (c.alone * kt + c.fixed);
+  return (float)(per_cu / 2) * (c.pair * kt + c.fixed) + (float)(per_cu % 2) * (c.alone * kt + c.fixed);
+}
+// The macro-tile with the lowest cost. A smaller one must promise 12 % over 256 x 256: with
+// several rounds of pairs on long reductions the estimates are up to that much too low
+// (8192 x 2048 x 10240: 304 estimated, 344 measured, 247 on 256 x 256).
+inline int pick_tile(long m, long n, long k, int am, int bm, bool paired, float* time = nullptr) {
+  const int cus = device_cus();
+  const long kt = cdiv(k, kFBK);
+  int best = kTile256;
+  float t = 0.88f * tile_time(kTile256, m, n, kt, am, bm, cus);
+  // A paired 64 x 64 tile would write 32-byte row pieces.
+  for (int i = 1; i < (paired ? kTile64 : kFastTiles); ++i) {
+    const float ti = tile_time(i, m, n, kt, am, bm, cus);
+    if (ti < t) {
+      best = i;
+      t = ti;
+    }
+  }
+  if (time) *time = best == kTile256 ? t / 0.88f : t;
+  return best;
+}
+
+template <class Cfg, int AM, int BMD, bool PAIRED, class Epi>
+int run_ring(GemmParams p, hipStream_t stream) {
+  const void* kern = reinterpret_cast<const void*>(&gemm_ring_kernel<Cfg, AM, BMD, PAIRED, Epi>);
+  if (int rc = ensure_lds(kern, Cfg::kLds)) return rc;
+  p.tiles_m = cdiv(p.M, Cfg::BM);
+  p.tiles_n = cdiv(PAIRED ? p.H : p.N, PAIRED ? Cfg::BN / 2 : Cfg::BN);
+  p.total_tiles = p.tiles_m * p.tiles_n;
+  p.k_tiles_per_split = cdiv(p.K, kFBK);
+  hipLaunchKernelGGL((gemm_ring_kernel<Cfg, AM, BMD, PAIRED, Epi>), dim3(p.total_tiles),
+                     dim3(Cfg::NT), Cfg::kLds, stream, p);
+  return hip_check(hipGetLastError(), "gemm launch");
+}
+
+template <int AM, int BMD, bool PAIRED, class Epi>
+int run_ring_tile(const GemmParams& p, int tile, hipStream_t s) {
+  switch (tile) {
+    case kTile128x2: return run_ring<Ring128x2, AM, BMD, PAIRED, Epi>(p, s);
+    case kTile128x1: return run_ring<Ring128x1, AM, BMD, PAIRED, Epi>(p, s);
+    case kTile64x128: return run_ring<Ring64x128, AM, BMD, PAIRED, Epi>(p, s);
+    default:
+      if constexpr (!PAIRED) return run_ring<Ring64, AM, BMD, PAIRED, Epi>(p, s);
+  }
+  return set_error(kInvalid, "no GEMM macro-tile %d", tile);
+}
+
+// The fast path with the macro-tile picked by tile_time. MASK holds the operand layouts
+// (ab_bit) the smaller tiles are built for; the others run on 256 x 256 tiles.
+constexpr unsigned kMaskKRows = ab_bit(kKContig, kKContig) | ab_bit(kKContig, kMNContig);
+constexpr unsigned kMaskVector = kMaskKRows | ab_bit(kMNContig, kKContig) | ab_bit(kMNContig, kMNContig);
+template <unsigned MASK, bool PAIRED, class Epi>
+int dispatch_tiles(const GemmParams& p, int am, int bm, LaunchCfg cfg, hipStream_t s) {
+  const int tile = (MASK & ab_bit(am, bm)) ? pick_tile(p.M, p.N, p.K, am, bm, PAIRED) : kTile256;
+  if (tile == kTile256) return dispatch_fast<PAIRED, Epi>(p, am, bm, cfg, s);
+#define WS_RING(A_, B_)                                                          \
+  if constexpr ((MASK & ab_bit(A_, B_)) != 0)                                    \
+    if (am == A_ && bm == B_) return run_ring_tile<A_, B_, PAIRED, Epi>(p, tile, s);
+  WS_RING(0, 0) WS_RING(0, 1) WS_RING(1, 0) WS_RING(1, 1)
+#undef WS_RING
+  return set_error(kInvalid, "no GEMM instantiation for operand layouts (%d, %d)", am, bm);
 }
 
 }  // namespace ws

@@ -52,7 +52,7 @@ extern "C" int ws_mm(const void* a, int64_t a_s0, int64_t a_s1, const void* b, i
   LaunchCfg cfg{algorithm != 0, 1};
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (tile == kTileLarge && fast_ok(p, am, bm, false))
-    return dispatch_fast<false, FEpiStore<false, false>>(p, am, bm, cfg, s);
+    return dispatch_tiles<kMaskVector, false, FEpiStore<false, false>>(p, am, bm, cfg, s);
   if (tile == kTileLarge)
     return dispatch<kMaskMM, WS_TILE_ARGS_LARGE, false, EpiStore<false, false>>(p, am, bm, cfg, s);
   return dispatch<kMaskMM, WS_TILE_ARGS_SMALL, false, EpiStore<false, false>>(p, am, bm, cfg, s);
@@ -88,7 +88,7 @@ extern "C" int ws_swiglu_mm(const void* a, int64_t a_s0, int64_t a_s1, const voi
   LaunchCfg cfg{algorithm != 0, 1};
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (tile == kTileLarge && fast_ok(p, am, bm, true))
-    return dispatch_fast<true, FEpiSwiglu>(p, am, bm, cfg, s);
+    return dispatch_tiles<kMaskKRows, true, FEpiSwiglu>(p, am, bm, cfg, s);
   if (tile == kTileLarge)
     return dispatch<kMaskKK | kMaskGG, WS_TILE_ARGS_LARGE, true, EpiSwiglu>(p, am, bm, cfg, s);
   return dispatch<kMaskKK | kMaskGG, WS_TILE_ARGS_SMALL, true, EpiSwiglu>(p, am, bm, cfg, s);
