@@ -907,8 +907,10 @@ static __global__ void __launch_bounds__(256) transpose_bf16_kernel(
 // written as eight 16-byte column pieces after an in-register transpose (one byte
 // permutation per output word). The 64 lanes of a wave cover a 64 x 64 tile (lane
 // 8 * br + bc holds block (br, bc)), so every load instruction reads, and every store
-// writes, eight whole 128-byte lines. No LDS and no barrier. Streaming (non-temporal)
-// stores: 5.5 -> 6.0-6.4 TB/s on the weight shapes of the layer step.
+// writes, eight whole 128-byte lines. No LDS and no barrier. Plain stores: streaming ones
+// make this kernel 2-3 us faster (5.5 -> 6.0-6.4 TB/s) and the GEMM that reads the copy next
+// much slower, since it then fetches the copy from HBM for every XCD (4096 x 1280 x 6400 on
+// 128 x 128 tiles: 75 us after plain stores, 113 us after streaming ones).
 static __global__ void __launch_bounds__(256) transpose_bf16_reg_kernel(
     const unsigned short* __restrict__ in, long ld_in, unsigned short* __restrict__ out,
     int rows, int cols) {
@@ -929,7 +931,7 @@ static __global__ void __launch_bounds__(256) transpose_bf16_reg_kernel(
     for (int p = 0; p < 4; ++p)
       o[p] = __builtin_amdgcn_perm(w[2 * p + 1][q >> 1], w[2 * p][q >> 1],
                                    (q & 1) ? 0x07060302u : 0x05040100u);
-    __builtin_nontemporal_store(o, reinterpret_cast<u32x4_t*>(out + (long)(c + q) * rows + r));
+    *reinterpret_cast<u32x4_t*>(out + (long)(c + q) * rows + r) = o;
   }
 }
 

@@ -57,8 +57,8 @@ def _check_buffer(t: torch.Tensor, shape: tuple, dtype: torch.dtype, device: tor
         raise ValueError(f"{name} must have a unit column stride")
 
 
-# Rows of A from which a transposed copy of an N-contiguous B pays for itself: the copy
-# moves 4 |B| bytes once, the GEMM reads B's tiles once per 256-row block of A.
+# Rows of A from which a transposed copy of an N-contiguous B can pay for itself: the copy
+# moves 4 |B| bytes once, the GEMM reads B's tiles once per row block of A.
 TRANSPOSE_MIN_ROWS = 1024
 
 
@@ -86,13 +86,29 @@ def k_contiguous_b(b: torch.Tensor, rows_a: int) -> torch.Tensor:
     return b
 
 
+def gemm_b(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """B [K, N] as the GEMM of ``a`` [M, K] best reads it: ``k_contiguous_b``'s copy, or B
+    itself where the vector loaders read an N-contiguous B directly at no loss: beside a
+    token-major A (a weight gradient's dY.T: both operands go through the same transposing
+    loop; 10240 x 2048 x 8192 takes 421 us with a copied B, 300 without) and for products
+    that the library expects to gain less than the copy costs (``ws_mm_copy_pays``). Same
+    bits."""
+    k, n = b.shape
+    if b.stride(1) == 1 and n % 8 == 0 and b.stride(0) % 8 == 0 and b.data_ptr() % 16 == 0:
+        token_major = (a.stride(0) == 1 and a.shape[0] % 8 == 0 and a.stride(1) % 8 == 0
+                       and a.data_ptr() % 16 == 0)
+        if token_major or not _hip.query("ws_mm_copy_pays", a.shape[0], n, k):
+            return b
+    return k_contiguous_b(b, a.shape[0])
+
+
 def mm(a: torch.Tensor, b: torch.Tensor, algorithm: str = "tiled", tile: int = 0) -> torch.Tensor:
     """r(a @ b) with the HIP GEMM; `tile` 0 = 256x256, 1 = 128x128."""
     _check_bf16_cuda(a, b)
     if a.ndim != 2 or b.ndim != 2 or a.shape[1] != b.shape[0]:
         raise ValueError(f"Expected a [M, K] and b [K, N], got {list(a.shape)} and {list(b.shape)}")
     if tile == 0:
-        b = k_contiguous_b(b, a.shape[0])
+        b = gemm_b(a, b)
     m, k = a.shape
     n = b.shape[1]
     out = torch.empty((m, n), dtype=torch.bfloat16, device=a.device)
@@ -110,8 +126,7 @@ def dgrad_mm(grad: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     This library's GEMM (``ws_mm``, FP32 accumulation, one BF16 rounding) on the
     persistent grid (one workgroup per CU looping over the tiles: 2.5-3.5 % faster than a
     workgroup per tile at 16384 x 2048 x 9216 / x 11264, bit-identical), with the weight
-    first copied K-contiguous by the HIP transpose kernel (``k_contiguous_b``) when grad
-    has enough rows to amortize the copy.
+    first copied K-contiguous by the HIP transpose kernel where that pays (``gemm_b``).
     """
     _check_bf16_cuda(grad, weight)
     if grad.dim() != 2 or weight.dim() != 2 or grad.shape[1] != weight.shape[0]:
@@ -233,7 +248,7 @@ def swiglu_backward_mm(grad: torch.Tensor, down_weight: torch.Tensor, packed: to
     if out is None:
         out = torch.empty((m, 2 * h), dtype=torch.bfloat16, device=grad.device)
     _check_buffer(out, (m, 2 * h), torch.bfloat16, grad.device, "out")
-    down_weight = k_contiguous_b(down_weight, m)
+    down_weight = gemm_b(grad, down_weight)
     _hip.call("ws_swiglu_backward_mm", grad.data_ptr(), grad.stride(0), grad.stride(1),
               down_weight.data_ptr(), down_weight.stride(0), down_weight.stride(1),
               packed.data_ptr(), out.data_ptr(), m, h, k, int(eager_rounding), _hip.stream(grad))
