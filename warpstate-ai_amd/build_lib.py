@@ -1,4 +1,5 @@
-"""Compile ``csrc/*.hip`` for gfx950 into ``lib/libwarpstate_hip.so``.
+"""Compile ``csrc/*.hip`` for gfx950 into ``lib/libwarpstate_hip.so``, and the operators'
+host-side autograd kernels (``csrc/autograd.cpp``) into ``lib/libwarpstate_autograd.so``.
 
 Every translation unit is compiled on each call (in parallel), then linked into a fresh
 library that atomically replaces the old one. Objects go to ``_build/``.
@@ -6,6 +7,7 @@ library that atomically replaces the old one. Objects go to ``_build/``.
 
 from __future__ import annotations
 
+import importlib.util
 import os
 import subprocess
 import sys
@@ -16,7 +18,9 @@ PACKAGE = Path(__file__).resolve().parent
 CSRC = PACKAGE / "csrc"
 BUILD = PACKAGE / "_build"
 LIBRARY = PACKAGE / "lib" / "libwarpstate_hip.so"
+AUTOGRAD = PACKAGE / "lib" / "libwarpstate_autograd.so"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+CXX = os.environ.get("CXX", "g++")
 ARCH = "gfx950"
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
@@ -39,6 +43,21 @@ def _compile(source: Path) -> Path:
     return obj
 
 
+def _build_autograd() -> Path:
+    """The C++ autograd kernels: host code against PyTorch's headers, no device code."""
+    torch_dir = Path(importlib.util.find_spec("torch").origin).parent
+    include = torch_dir / "include"
+    staging = AUTOGRAD.with_name(AUTOGRAD.name + ".tmp")
+    cmd = [CXX, "-O2", "-std=c++17", "-fPIC", "-shared", f"-I{include}",
+           f"-I{include / 'torch' / 'csrc' / 'api' / 'include'}", str(CSRC / "autograd.cpp"),
+           "-o", str(staging), f"-L{torch_dir / 'lib'}", "-ltorch", "-ltorch_cpu", "-lc10"]
+    result = subprocess.run(cmd, capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError(f"{CXX} failed for autograd.cpp:\n{result.stderr}")
+    os.replace(staging, AUTOGRAD)
+    return AUTOGRAD
+
+
 def build(jobs: int | None = None) -> Path:
     sources = sorted(CSRC.glob("*.hip"))
     if not sources:
@@ -47,7 +66,9 @@ def build(jobs: int | None = None) -> Path:
     LIBRARY.parent.mkdir(exist_ok=True)
     jobs = jobs or min(len(sources), max(1, min(os.cpu_count() or 1, 16)))
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        autograd = pool.submit(_build_autograd)
         objects = list(pool.map(_compile, sources))
+        autograd.result()
     staging = LIBRARY.with_name(LIBRARY.name + ".tmp")
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-o", str(staging), *map(str, objects)]
     result = subprocess.run(cmd, capture_output=True, text=True)

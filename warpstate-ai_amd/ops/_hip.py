@@ -15,6 +15,7 @@ from pathlib import Path
 import torch
 
 LIBRARY_PATH = Path(__file__).resolve().parents[1] / "lib" / "libwarpstate_hip.so"
+AUTOGRAD_PATH = LIBRARY_PATH.with_name("libwarpstate_autograd.so")
 
 _c_void_p = ctypes.c_void_p
 _i64 = ctypes.c_int64
@@ -119,6 +120,24 @@ def library() -> ctypes.CDLL:
     return _library
 
 
+_autograd_loaded = False
+
+
+def load_autograd() -> None:
+    """Register the native autograd kernels of the row and fused training operators on CUDA
+    (``csrc/autograd.cpp``), once; raise if the kernels are built and these are not. Before
+    anything is built the operators import with their Python autograd formulas."""
+    global _autograd_loaded
+    with _lock:
+        if _autograd_loaded or not LIBRARY_PATH.exists():
+            return
+        if not AUTOGRAD_PATH.exists():
+            raise RuntimeError(f"native autograd kernels not built: {AUTOGRAD_PATH} is missing "
+                               "(run __graft_entry__.build())")
+        torch.ops.load_library(str(AUTOGRAD_PATH))
+        _autograd_loaded = True
+
+
 def call(name: str, *args) -> None:
     """Invoke a status-returning entry point; raise RuntimeError on failure."""
     lib = library()
@@ -134,7 +153,10 @@ def query(name: str, *args) -> int:
 
 def stream(tensor: torch.Tensor) -> int:
     """HIP stream handle of the calling thread's current stream on the tensor's device."""
-    return torch.cuda.current_stream(tensor.device).cuda_stream
+    index = tensor.get_device()
+    if index < 0:  # not a GPU tensor: PyTorch's own error
+        return torch.cuda.current_stream(tensor.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def ptr(tensor: torch.Tensor | None) -> int | None:

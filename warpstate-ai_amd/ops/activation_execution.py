@@ -117,6 +117,8 @@ def _rms_autograd(ctx, grad, _grad_rstd):
 
 bf16_rmsnorm.register_autograd(_rms_autograd, setup_context=_rms_setup)
 
+_hip.load_autograd()
+
 
 _MODES = {"baseline": (), "swiglu": ("swiglu",), "rmsnorm": ("rmsnorm",),
           "all": ("swiglu", "rmsnorm")}

@@ -47,6 +47,7 @@ from __future__ import annotations
 
 import torch
 
+from ops import _hip
 from ops import fused_execution as fx
 from ops._patching import bf16_autocast_training
 
@@ -290,6 +291,8 @@ def _swiglu_mlp_autograd(ctx, dout, _dpacked, _dact, _dwug, _dwd):
 
 
 fused_swiglu_mlp.register_autograd(_swiglu_mlp_autograd, setup_context=_swiglu_mlp_setup)
+
+_hip.load_autograd()
 
 
 def _rows_bf16(x: Tensor) -> Tensor:
