@@ -225,6 +225,12 @@ int ws_mm_store_f32(const void* a, int64_t a_s0, int64_t a_s1, const void* b, in
 int ws_mm_store_f32_group(const ws_accumulate_problem* problems, int count, int64_t k,
                           int round_bf16, float* workspace, void* stream);
 
+/* Or-ed into a leading dimension of the LM-head gradient calls (ld_dweight of
+ * ws_linear_ce_backward and ws_linear_ce_fused, ld_unit of ws_linear_ce_fused_backward):
+ * dweight is written instead of accumulated into, so that it needs no clearing and is not
+ * read before it is written. */
+#define WS_WRITE_DWEIGHT ((int64_t)1 << 62)
+
 /* Number of per-row partials (floats per row of part_max / part_sum) for `vocab`. */
 int64_t ws_linear_ce_parts(int64_t vocab);
 

@@ -797,14 +797,27 @@ static __global__ void __launch_bounds__(256) scale_bf16_rows_kernel(
   out[r * ld_out + c] = to_bf16_bits(scale * bf16_bits_to_f32(in[r * ld_in + c]));
 }
 
-// acc += g * x elementwise over n FP32 values.
-static __global__ void __launch_bounds__(256) scale_add_f32_kernel(const float* __restrict__ g,
-                                                             const float* __restrict__ x,
-                                                             float* __restrict__ acc, long n,
-                                                             const int* __restrict__ run_if) {
+// acc += g * x elementwise over n FP32 values, or acc = g * x (WRITE; acc is not read), four
+// values per thread (16-byte pieces when `vec`: both pointers 16-byte aligned). HBM-bound.
+template <bool WRITE>
+static __global__ void __launch_bounds__(256) scale_f32_kernel(const float* __restrict__ g,
+                                                               const float* __restrict__ x,
+                                                               float* __restrict__ acc, long n,
+                                                               const int* __restrict__ run_if,
+                                                               int vec) {
   if (run_if != nullptr && *run_if == 0) return;
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) acc[i] += *g * x[i];
+  const float scale = *g;
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (vec && i + 3 < n) {
+    const f32x4_t v = *reinterpret_cast<const f32x4_t*>(x + i);
+    f32x4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = scale * v[e];
+    if (!WRITE) o = *reinterpret_cast<const f32x4_t*>(acc + i) + o;
+    *reinterpret_cast<f32x4_t*>(acc + i) = o;
+    return;
+  }
+  for (long j = i; j < n && j < i + 4; ++j) acc[j] = WRITE ? scale * x[j] : acc[j] + scale * x[j];
 }
 
 // exact[0] = 1 when g is +-2^e with |e| <= 32 (a normal FP32 number with an all-zero

@@ -97,6 +97,9 @@ def problem_table(rows) -> ctypes.Array:
     return (AccumulateProblem * len(rows))(*[AccumulateProblem(*r) for r in rows])
 
 
+# WS_WRITE_DWEIGHT of include/warpstate_hip.h.
+WRITE_DWEIGHT = 1 << 62
+
 _lock = threading.Lock()
 _library = None
 

@@ -470,8 +470,6 @@ def linear_cross_entropy_forward(hidden: torch.Tensor, weight: torch.Tensor,
         # Kept for the backward's two-pass fallback (an upstream gradient that is not a
         # power of two).
         state.weight_t = weight_t
-        if state.dweight_unit is not None:
-            state.dweight_unit.zero_()
         _hip.call("ws_linear_ce_fused", hidden.data_ptr(), hidden.stride(0), weight.data_ptr(),
                   weight.stride(0), _hip.ptr(weight_t), targets.data_ptr(), rows, vocab, d,
                   state.part_max.data_ptr(), state.part_sum.data_ptr(),
@@ -479,7 +477,8 @@ def linear_cross_entropy_forward(hidden: torch.Tensor, weight: torch.Tensor,
                   state.mean.data_ptr(), state.count.data_ptr(), workspace.data_ptr(),
                   state.chunk_rows, state.dhidden_unit.data_ptr(), state.dhidden_unit.stride(0),
                   _hip.ptr(state.dweight_unit),
-                  0 if state.dweight_unit is None else state.dweight_unit.stride(0),
+                  0 if state.dweight_unit is None
+                  else state.dweight_unit.stride(0) | _hip.WRITE_DWEIGHT,
                   _hip.stream(hidden))
         return state
     _hip.call("ws_linear_ce_forward", hidden.data_ptr(), hidden.stride(0), weight.data_ptr(),
@@ -494,11 +493,13 @@ def linear_cross_entropy_backward(hidden: torch.Tensor, weight: torch.Tensor,
                                   targets: torch.Tensor, state: CrossEntropyState,
                                   grad_mean: torch.Tensor,
                                   out: torch.Tensor | None = None,
-                                  weight_grad: torch.Tensor | None = None) -> torch.Tensor:
+                                  weight_grad: torch.Tensor | None = None,
+                                  accumulate: bool = True) -> torch.Tensor:
     """dHidden [rows, d] BF16 of ``mean`` given its FP32 scalar gradient.
 
     ``weight_grad`` (FP32 [vocab, d], unit column stride), when given, accumulates the tied
-    head weight's gradient chunk by chunk: weight_grad += f32(r(G_chunk^T @ hidden_chunk)).
+    head weight's gradient chunk by chunk: weight_grad += f32(r(G_chunk^T @ hidden_chunk));
+    with ``accumulate=False`` it is written instead (its contents are not read).
     """
     _check_ce(hidden, weight, targets)
     rows, d = hidden.shape
@@ -513,6 +514,7 @@ def linear_cross_entropy_backward(hidden: torch.Tensor, weight: torch.Tensor,
     if weight_grad is not None:
         _check_buffer(weight_grad, (vocab, d), torch.float32, hidden.device, "weight_grad",
                       contiguous=state.fused)
+    write = 0 if accumulate or weight_grad is None else _hip.WRITE_DWEIGHT
     if state.fused:
         if state.d != d:
             raise ValueError(f"The fused CrossEntropyState was built for d={state.d}, not {d}")
@@ -522,7 +524,8 @@ def linear_cross_entropy_backward(hidden: torch.Tensor, weight: torch.Tensor,
                   weight.data_ptr(), weight.stride(0), _hip.ptr(state.weight_t),
                   targets.data_ptr(), state.lse.data_ptr(), state.count.data_ptr(),
                   grad_mean.data_ptr(), rows, vocab, d, state.backward_workspace(d).data_ptr(),
-                  state.chunk_rows, state.dhidden_unit.data_ptr(), state.dhidden_unit.stride(0),
+                  state.chunk_rows, state.dhidden_unit.data_ptr(),
+                  state.dhidden_unit.stride(0) | write,
                   None if weight_grad is None else state.dweight_unit.data_ptr(),
                   out.data_ptr(), out.stride(0), _hip.ptr(weight_grad), _hip.stream(hidden))
         return out
@@ -535,7 +538,7 @@ def linear_cross_entropy_backward(hidden: torch.Tensor, weight: torch.Tensor,
               grad_mean.data_ptr(), rows, vocab, d, workspace.data_ptr(), state.chunk_rows,
               out.data_ptr(), out.stride(0),
               None if weight_grad is None else weight_grad.data_ptr(),
-              0 if weight_grad is None else weight_grad.stride(0), _hip.ptr(state.logits),
+              0 if weight_grad is None else weight_grad.stride(0) | write, _hip.ptr(state.logits),
               _hip.stream(hidden))
     return out
 
@@ -588,10 +591,10 @@ class LinearCrossEntropy(torch.autograd.Function):
         if grad_mean is None:
             grad_mean = torch.zeros((), dtype=torch.float32, device=h.device)
         want_h, want_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        weight_grad = (torch.zeros(w.shape, dtype=torch.float32, device=w.device)
+        weight_grad = (torch.empty(w.shape, dtype=torch.float32, device=w.device)
                        if want_w else None)
         dh = linear_cross_entropy_backward(h, w, targets, ctx.state, grad_mean,
-                                           weight_grad=weight_grad)
+                                           weight_grad=weight_grad, accumulate=False)
         hidden_dtype, weight_dtype = ctx.dtypes
         return (dh.to(hidden_dtype) if want_h else None,
                 weight_grad.to(weight_dtype) if want_w else None, None, None, None)
