@@ -220,6 +220,55 @@ __global__ void __launch_bounds__(256) sk_accum_kernel(const float* __restrict__
   }
 }
 
+// How one FP32 weight gradient runs: on 256 x 256 tiles (balanced or evenly split) or on a
+// ring macro-tile with `splits` k-slices.
+struct WgradPlan {
+  int tile, splits;
+  float time;
+};
+
+// Reducing `slices` FP32 slices of an [m, n] output into G (read too unless it is stored).
+float reduce_time(long m, long n, long slices, bool store) {
+  return 4.0f + 4.0f * (float)m * (float)n * (float)(slices + (store ? 1 : 2)) / 5.5e6f;
+}
+// The balanced plan: whole rounds, the shared tiles' pieces and their ordered sum.
+float balanced_time(const BalancedPlan& b, int workers) {
+  const float alone = tile_cost(kTile256, kMNContig, kMNContig).alone;
+  const float fixed = tile_cost(kTile256, kMNContig, kMNContig).fixed;
+  const float loop = alone * (float)b.tiles * (float)b.k_tiles / (float)workers;
+  const float rounds = fixed * (float)(b.dp_tiles / workers + (b.sk_tiles > 0));
+  return loop + rounds +
+         (b.sk_tiles ? 4.0f + 4.0f * kFBM * kFBN * (float)b.sk_tiles * (b.pieces + 2) / 5.5e6f : 0.0f);
+}
+// The cheapest way for a token-major gradient (both operands M/N-contiguous) whose caller
+// allows up to `splits` slices. The 256 x 256 schemes stay unless a smaller tile promises
+// 12 % more (launch.h). Measured, us: 6400 x 1280 x 4096 66 + 20 (two slices and their sum)
+// against 68 (128 x 128); 1280 x 4480 + 8960 x 1280 over 512 tokens 40 + 6 (balanced, one
+// launch) against 16 + 23; over 1999 tokens 85 + 13 against 36 + 56 (balanced kept).
+WgradPlan wgrad_plan(long m, long n, long k, int splits, bool store, int workers) {
+  const long kt = cdiv(k, kFBK);
+  const BalancedPlan b = balanced_plan(m, n, k, workers);
+  WgradPlan best{kTile256, splits, 0.0f};
+  if (splits <= 1 || b.sk_tiles == 0)
+    best.time = tile_time(kTile256, m, n, kt, kMNContig, kMNContig, workers);
+  else if (b.dp_tiles > 0)
+    best.time = balanced_time(b, workers);
+  else
+    best.time = tile_time(kTile256, m, n, cdiv(kt, splits), kMNContig, kMNContig, workers, splits) +
+                reduce_time(m, n, splits, store);
+  float limit = 0.88f * best.time;
+  for (int tile = kTile256 + 1; tile < kFastTiles; ++tile)
+    for (int s = 1; s <= splits; ++s) {
+      const float t = tile_time(tile, m, n, cdiv(kt, s), kMNContig, kMNContig, workers, s) +
+                      (s > 1 ? reduce_time(m, n, s, store) : 0.0f);
+      if (t < limit) {
+        best = WgradPlan{tile, s, t};
+        limit = t;
+      }
+    }
+  return best;
+}
+
 }  // namespace
 
 extern "C" int64_t ws_mm_accumulate_workspace_floats(int64_t m, int64_t n, int64_t k, int64_t splits) {
@@ -252,18 +301,24 @@ int mm_f32(const void* a, int64_t a_s0, int64_t a_s1, const void* b, int64_t b_s
   p.g = g;
   p.ldg = ldg;
   p.vec_out = (n % 4 == 0) && (ldg % 4 == 0) && al(g, 16);
+  const int workers = device_cus();
+  const bool fast = fast_ok(p, am, bm, false);
+  WgradPlan ring{kTile256, (int)splits, 0.0f};
+  if (fast && am == kMNContig && bm == kMNContig)
+    ring = wgrad_plan(m, n, k, splits > 1 && al(workspace, 16) ? (int)splits : 1,
+                      (acc & kAccStore) != 0, workers);
+  if (ring.tile != kTile256 && ring.splits == 1)
+    return run_ring_tile<kMNContig, kMNContig, false, FEpiAccF32<false>>(p, ring.tile, s);
   if (splits <= 1) {
-    if (fast_ok(p, am, bm, false))
+    if (fast)
       return dispatch_fast<false, FEpiAccF32<false>>(p, am, bm, LaunchCfg{0, 1}, s);
     return dispatch<kMaskMM, WS_TILE_ARGS_LARGE, false, EpiAccF32<false>>(p, am, bm,
                                                                                   LaunchCfg{0, 1}, s);
   }
-  const int workers = device_cus();
   const BalancedPlan plan = balanced_plan(m, n, k, workers);
-  const bool fast = fast_ok(p, am, bm, false);
-  if (fast && plan.sk_tiles == 0)  // whole rounds of tiles: nothing to split
+  if (ring.tile == kTile256 && fast && plan.sk_tiles == 0)  // whole rounds: nothing to split
     return dispatch_fast<false, FEpiAccF32<false>>(p, am, bm, LaunchCfg{0, 1}, s);
-  if (fast && plan.dp_tiles > 0 && al(workspace, 16)) {
+  if (ring.tile == kTile256 && fast && plan.dp_tiles > 0 && al(workspace, 16)) {
     // Balanced: whole rounds of tiles accumulate directly, the rest is shared stream-K.
     p.balanced = 1;
     p.dp_tiles = plan.dp_tiles;
@@ -288,7 +343,11 @@ int mm_f32(const void* a, int64_t a_s0, int64_t a_s1, const void* b, int64_t b_s
   p.ldg = n;
   p.split_stride = m * n;
   p.vec_out = (n % 4 == 0) && al(workspace, 16);
-  if (fast && p.vec_out) {
+  const int slices = ring.tile != kTile256 ? ring.splits : (int)splits;
+  if (ring.tile != kTile256) {
+    if (int rc = run_ring_tile<kMNContig, kMNContig, false, FEpiAccF32<true>>(p, ring.tile, s, slices))
+      return rc;
+  } else if (fast && p.vec_out) {
     if (int rc = dispatch_fast<false, FEpiAccF32<true>>(p, am, bm, LaunchCfg{0, (int)splits}, s))
       return rc;
   } else if (int rc = dispatch<kMaskMM, WS_TILE_ARGS_LARGE, false, EpiAccF32<true>>(
@@ -298,8 +357,7 @@ int mm_f32(const void* a, int64_t a_s0, int64_t a_s1, const void* b, int64_t b_s
   const int vec = (n % 4 == 0) && (ldg % 4 == 0) && al(g, 16) && al(workspace, 16);
   const long threads = vec ? m * n / 4 : m * n;
   hipLaunchKernelGGL(splitk_accum_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s,
-                     workspace, (int)splits, (long)(m * n), g, (long)ldg, (int)m, (int)n,
-                     acc, vec);
+                     workspace, slices, (long)(m * n), g, (long)ldg, (int)m, (int)n, acc, vec);
   return hip_check(hipGetLastError(), "split-K reduce launch");
 }
 
@@ -422,6 +480,16 @@ int mm_f32_group(const ws_accumulate_problem* problems, int count, int64_t k, in
     const int tm = cdiv(q.m, kFBM), tn = cdiv(q.n, kFBN);
     p.grp[i] = GemmMember{pi.a, pi.b, (int)q.m, (int)q.n, tm, tn, base, q.g, (long)q.ldg};
     base += tm * tn;
+  }
+  if (one_launch && am == kMNContig && bm == kMNContig) {
+    // Separate launches on smaller tiles where they promise more than the one launch.
+    float apart = 0.0f;
+    for (int i = 0; i < count; ++i) {
+      const long m = problems[i].m, n = problems[i].n;
+      apart += wgrad_plan(m, n, k, workspace ? auto_splits(m, n, k, workers) : 1,
+                          (acc & kAccStore) != 0, workers).time;
+    }
+    one_launch = apart >= 0.88f * balanced_time(plan, workers);
   }
   if (!one_launch) {
     for (int i = 0; i < count; ++i) {

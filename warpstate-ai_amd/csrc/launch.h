@@ -220,10 +220,12 @@ inline const TileCost& tile_cost(int tile, int am, int bm) {
   if (am == kKContig && bm == kKContig) return kk[tile];
   return (am == kMNContig && bm == kMNContig ? mnmn : kmn)[tile];
 }
-// An [m, n] output (n the packed width of a paired GEMM) over k_tiles k-tiles.
-inline float tile_time(int tile, long m, long n, long k_tiles, int am, int bm, int cus) {
+// An [m, n] output (n the packed width of a paired GEMM) over k_tiles k-tiles, or `copies` of
+// it (split-K slices of k_tiles each).
+inline float tile_time(int tile, long m, long n, long k_tiles, int am, int bm, int cus,
+                       long copies = 1) {
   const TileCost& c = tile_cost(tile, am, bm);
-  const long tiles = (long)cdiv(m, c.bm) * cdiv(n, c.bn), rounds = tiles / cus;
+  const long tiles = (long)cdiv(m, c.bm) * cdiv(n, c.bn) * copies, rounds = tiles / cus;
   const float kt = (float)k_tiles;
   if (tile == kTile256) {
     // With most CUs idle in the last round its tiles' loads meet less traffic.
@@ -256,26 +258,26 @@ inline int pick_tile(long m, long n, long k, int am, int bm, bool paired, float*
 }
 
 template <class Cfg, int AM, int BMD, bool PAIRED, class Epi>
-int run_ring(GemmParams p, hipStream_t stream) {
+int run_ring(GemmParams p, int splits, hipStream_t stream) {
   const void* kern = reinterpret_cast<const void*>(&gemm_ring_kernel<Cfg, AM, BMD, PAIRED, Epi>);
   if (int rc = ensure_lds(kern, Cfg::kLds)) return rc;
   p.tiles_m = cdiv(p.M, Cfg::BM);
   p.tiles_n = cdiv(PAIRED ? p.H : p.N, PAIRED ? Cfg::BN / 2 : Cfg::BN);
   p.total_tiles = p.tiles_m * p.tiles_n;
-  p.k_tiles_per_split = cdiv(p.K, kFBK);
-  hipLaunchKernelGGL((gemm_ring_kernel<Cfg, AM, BMD, PAIRED, Epi>), dim3(p.total_tiles),
+  p.k_tiles_per_split = cdiv(cdiv(p.K, kFBK), splits);
+  hipLaunchKernelGGL((gemm_ring_kernel<Cfg, AM, BMD, PAIRED, Epi>), dim3(p.total_tiles, splits),
                      dim3(Cfg::NT), Cfg::kLds, stream, p);
   return hip_check(hipGetLastError(), "gemm launch");
 }
 
 template <int AM, int BMD, bool PAIRED, class Epi>
-int run_ring_tile(const GemmParams& p, int tile, hipStream_t s) {
+int run_ring_tile(const GemmParams& p, int tile, hipStream_t s, int splits = 1) {
   switch (tile) {
-    case kTile128x2: return run_ring<Ring128x2, AM, BMD, PAIRED, Epi>(p, s);
-    case kTile128x1: return run_ring<Ring128x1, AM, BMD, PAIRED, Epi>(p, s);
-    case kTile64x128: return run_ring<Ring64x128, AM, BMD, PAIRED, Epi>(p, s);
+    case kTile128x2: return run_ring<Ring128x2, AM, BMD, PAIRED, Epi>(p, splits, s);
+    case kTile128x1: return run_ring<Ring128x1, AM, BMD, PAIRED, Epi>(p, splits, s);
+    case kTile64x128: return run_ring<Ring64x128, AM, BMD, PAIRED, Epi>(p, splits, s);
     default:
-      if constexpr (!PAIRED) return run_ring<Ring64, AM, BMD, PAIRED, Epi>(p, s);
+      if constexpr (!PAIRED) return run_ring<Ring64, AM, BMD, PAIRED, Epi>(p, splits, s);
   }
   return set_error(kInvalid, "no GEMM macro-tile %d", tile);
 }
