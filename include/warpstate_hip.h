@@ -86,7 +86,7 @@ int ws_rmsnorm_forward(const void* x, const float* weight, void* y, float* rstd,
                        int64_t d, float eps, int eager_rounding, void* stream);
 
 /* Floats of the `partial` workspace ws_rmsnorm_backward needs: one partial row of d floats
- * per 32 rows up to d = 2048, per 4 to 32 rows (depending on the row count) above. */
+ * per 8 to 32 rows up to d = 2048, per 4 to 32 rows above, depending on the row count. */
 int64_t ws_rmsnorm_backward_partial_floats(int64_t rows, int64_t d);
 
 /* RMSNorm backward: dx [rows, d] BF16 and dweight [d] FP32 from x, weight, rstd and a

@@ -119,8 +119,8 @@ static __global__ void __launch_bounds__(256) rmsnorm_rows_reg_kernel(
 // and the weight-gradient partial sum over this block's rows of r?(dy z) (r? = BF16
 // rounding when eager). Rows of up to 2048 columns: one wave per row, 16-byte loads: lane
 // l owns columns 8 l + 512 s (s < SEGS), and keeps its x and dy chunks in registers between
-// the two passes over the row. A block of kRmsWaves waves takes kRmsRowsPerBlock
-// consecutive rows (wave w the rows w, w + kRmsWaves, ...); each wave's weight-gradient
+// the two passes over the row. A block of kRmsWaves waves takes `rpb` consecutive rows (at
+// most kRmsRowsPerBlock; wave w the rows w, w + kRmsWaves, ...); each wave's weight-gradient
 // partial builds up in its own LDS row, and the waves' rows are added in wave order into
 // one partial row per block. Wider rows take the block-per-row kernels below.
 constexpr int kRmsRowsPerBlock = 32;
@@ -146,7 +146,8 @@ template <int SEGS, bool EAGER>
 static __global__ void __launch_bounds__(64 * kRmsWaves) __attribute__((amdgpu_waves_per_eu(4)))
 rmsnorm_bwd_kernel(const unsigned short* __restrict__ x, const float* __restrict__ w,
                    const float* __restrict__ rstd, const unsigned short* __restrict__ dy,
-                   unsigned short* __restrict__ dx, float* __restrict__ dw_part, int rows, int D) {
+                   unsigned short* __restrict__ dx, float* __restrict__ dw_part, int rows, int D,
+                   int rpb) {
   extern __shared__ float lds_part[];  // [kRmsWaves][D] partials, then [D] weight
   // The wave index as a scalar, so that row addresses are scalar bases plus one lane offset.
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -163,7 +164,7 @@ rmsnorm_bwd_kernel(const unsigned short* __restrict__ x, const float* __restrict
   }
   __syncthreads();
 
-  const int row_end = min(rows, (blockIdx.x + 1) * kRmsRowsPerBlock);
+  const int row_end = min(rows, (blockIdx.x + 1) * rpb);
   // One row ahead: the next row's x and dy are requested before this row's reduction.
   // (row is wave-uniform: the row bases are scalar and each lane adds its column offset.)
   auto load = [&](int row, u32x4_t (&xv)[SEGS], u32x4_t (&gv)[SEGS]) {
@@ -195,8 +196,8 @@ rmsnorm_bwd_kernel(const unsigned short* __restrict__ x, const float* __restrict
     }
   };
   u32x4_t xn[SEGS], gn[SEGS];
-  load(blockIdx.x * kRmsRowsPerBlock + wave, xn, gn);
-  for (int row = blockIdx.x * kRmsRowsPerBlock + wave; row < row_end; row += kRmsWaves) {
+  load(blockIdx.x * rpb + wave, xn, gn);
+  for (int row = blockIdx.x * rpb + wave; row < row_end; row += kRmsWaves) {
     const float r = rstd[row];
     u32x4_t xv[SEGS], gv[SEGS];
 #pragma unroll
@@ -262,13 +263,13 @@ template <bool EAGER>
 static __global__ void __launch_bounds__(64 * kRmsWaves) rmsnorm_bwd_generic_kernel(
     const unsigned short* __restrict__ x, const float* __restrict__ w,
     const float* __restrict__ rstd, const unsigned short* __restrict__ dy,
-    unsigned short* __restrict__ dx, float* __restrict__ dw_part, int rows, int D) {
+    unsigned short* __restrict__ dx, float* __restrict__ dw_part, int rows, int D, int rpb) {
   extern __shared__ float lds_part[];  // [kRmsWaves][D]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float* mine = lds_part + wave * D;
   for (int c = lane; c < D; c += 64) mine[c] = 0.0f;
-  const int row_end = min(rows, (blockIdx.x + 1) * kRmsRowsPerBlock);
-  for (int row = blockIdx.x * kRmsRowsPerBlock + wave; row < row_end; row += kRmsWaves) {
+  const int row_end = min(rows, (blockIdx.x + 1) * rpb);
+  for (int row = blockIdx.x * rpb + wave; row < row_end; row += kRmsWaves) {
     const float r = rstd[row];
     const unsigned short* xr = x + (long)row * D;
     const unsigned short* gr = dy + (long)row * D;

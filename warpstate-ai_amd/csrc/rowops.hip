@@ -73,12 +73,21 @@ extern "C" int ws_rmsnorm_forward(const void* x, const float* weight, void* y, f
                              static_cast<hipStream_t>(stream));
 }
 
-// Rows per block of the RMSNorm backward: 32 for rows of up to 2048 columns (8 waves, one
-// row each at a time); for wider rows (one row per block at a time) the largest power of two
-// from 4 to 32 that still gives at least 512 blocks (measured against 256 and 1024 at
-// 4096 to 8192 columns: 512 blocks was fastest or tied at every shape).
+// Rows per block of the RMSNorm backward. Rows of up to 2048 columns (8 waves, one row each
+// at a time): 32, or the fewer of 8 and 16 whose partials fit the static scratch array where
+// 32 would leave most compute units idle (at most 8192 rows; both calls, us: 512 x 1280 16.4
+// -> 8.8, 2048 x 1280 17.7 -> 10.1, 4096 x 2048 23.7 -> 18.1, 8192 x 1280 22.1 either way);
+// below 64 rows one or two blocks. For wider rows (one row per block at a time) the largest
+// power of two from 4 to 32 that still gives at least 512 blocks (measured against 256 and
+// 1024 at 4096 to 8192 columns: 512 blocks was fastest or tied at every shape).
+constexpr int64_t kStaticPartialFloats = 1L << 20;  // 4 MiB: rows x d up to 2^25 at d % 8 == 0
 static int rms_rows_per_block(int64_t rows, int64_t d) {
-  if (d <= 2048) return kRmsRowsPerBlock;
+  if (d <= 2048) {
+    if (rows >= 64 && rows <= 8192)
+      for (int rpb = 8; rpb < kRmsRowsPerBlock; rpb *= 2)
+        if (cdiv(rows, rpb) * d <= kStaticPartialFloats) return rpb;
+    return kRmsRowsPerBlock;
+  }
   int rpb = 4;
   while (rpb < 32 && rows / (2 * rpb) >= 512) rpb *= 2;
   return rpb;
@@ -95,10 +104,11 @@ static int launch_rms_bwd(const void* x, const float* weight, const float* rstd,
   const int lds = (kRmsWaves + (SEGS > 0 ? 1 : 0)) * d * (int)sizeof(float);
   auto launch = [&](auto kernel) {
     if (int rc = ensure_lds(reinterpret_cast<const void*>(kernel), lds)) return rc;
-    hipLaunchKernelGGL(kernel, dim3(cdiv(rows, kRmsRowsPerBlock)), dim3(64 * kRmsWaves), lds, s,
+    const int rpb = rms_rows_per_block(rows, d);
+    hipLaunchKernelGGL(kernel, dim3(cdiv(rows, rpb)), dim3(64 * kRmsWaves), lds, s,
                        static_cast<const unsigned short*>(x), weight, rstd,
                        static_cast<const unsigned short*>(grad), static_cast<unsigned short*>(dx),
-                       partial, rows, d);
+                       partial, rows, d, rpb);
     return hip_check(hipGetLastError(), "rmsnorm backward launch");
   };
   if constexpr (SEGS == 0)
@@ -181,7 +191,6 @@ extern "C" int ws_rmsnorm_backward(const void* x, const float* weight, const flo
 // the array needs no clearing; calls that overlap on one GPU share it and race.
 namespace {
 
-constexpr long kStaticPartialFloats = 1L << 20;  // 4 MiB: rows x d up to 2^25 at d % 8 == 0
 constexpr int kStaticMaxWidth = 8192;  // the widest row any RMSNorm backward kernel takes
 __device__ __align__(256) float scratch[kStaticPartialFloats];
 
