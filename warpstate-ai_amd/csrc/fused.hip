@@ -80,7 +80,7 @@ extern "C" int ws_rmsnorm_gate_mm(const void* x, int64_t x_s0, const float* norm
   p.gate_hi = (int)gate_end;
   int am = operand_mode(p.a, m, k, 256), bm = operand_mode(p.b, n, k, 256);
   if (fast_ok(p, am, bm, false))
-    return dispatch_tiles<kMaskKRows, false, FEpiStore<true, false>>(p, am, bm, kFusedCfg, s);
+    return dispatch_tiles<kMaskKRows, false, FEpiStore<true, false>>(p, am, bm, kFusedCfg, s, kEpiSigmoid);
   return dispatch<kMaskMM, WS_TILE_ARGS_LARGE, false, EpiStore<true, false>>(p, am, bm,
                                                                                    LaunchCfg{0, 1}, s);
 }
@@ -132,7 +132,7 @@ extern "C" int ws_swiglu_backward_mm(const void* grad, int64_t g_s0, int64_t g_s
   int am = operand_mode(p.a, m, k, 256), bm = operand_mode(p.b, h, k, 256);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (fast_ok(p, am, bm, false))
-    return dispatch_tiles<kMaskKRows, false, FEpiSwigluBwd>(p, am, bm, kFusedCfg, s);
+    return dispatch_tiles<kMaskKRows, false, FEpiSwigluBwd>(p, am, bm, kFusedCfg, s, kEpiSwigluBwd);
   constexpr unsigned mask = kMaskKK | ab_bit(kKContig, kMNContig) | kMaskGG;
   return dispatch<mask, WS_TILE_ARGS_LARGE, false, EpiSwigluBwd>(
       p, am, bm, LaunchCfg{0, 1}, s);
@@ -232,35 +232,36 @@ float reduce_time(long m, long n, long slices, bool store) {
   return 4.0f + 4.0f * (float)m * (float)n * (float)(slices + (store ? 1 : 2)) / 5.5e6f;
 }
 // The balanced plan: whole rounds, the shared tiles' pieces and their ordered sum.
-float balanced_time(const BalancedPlan& b, int workers) {
+float balanced_time(const BalancedPlan& b, bool store, int workers) {
   const float alone = tile_cost(kTile256, kMNContig, kMNContig).alone;
   const float fixed = tile_cost(kTile256, kMNContig, kMNContig).fixed;
   const float loop = alone * (float)b.tiles * (float)b.k_tiles / (float)workers;
-  const float rounds = fixed * (float)(b.dp_tiles / workers + (b.sk_tiles > 0));
+  const float rounds = (fixed + (store ? kEpiF32 : kEpiF32Add)) * (float)(b.dp_tiles / workers) +
+                       (b.sk_tiles ? fixed + kEpiF32 : 0.0f);
   return loop + rounds +
          (b.sk_tiles ? 4.0f + 4.0f * kFBM * kFBN * (float)b.sk_tiles * (b.pieces + 2) / 5.5e6f : 0.0f);
 }
 // The cheapest way for a token-major gradient (both operands M/N-contiguous) whose caller
 // allows up to `splits` slices. The 256 x 256 schemes stay unless a smaller tile promises
-// 12 % more (launch.h). Measured, us: 6400 x 1280 x 4096 66 + 20 (two slices and their sum)
+// 10 % more. Measured, us: 6400 x 1280 x 4096 66 + 20 (two slices and their sum)
 // against 68 (128 x 128); 1280 x 4480 + 8960 x 1280 over 512 tokens 40 + 6 (balanced, one
 // launch) against 16 + 23; over 1999 tokens 85 + 13 against 36 + 56 (balanced kept).
 WgradPlan wgrad_plan(long m, long n, long k, int splits, bool store, int workers) {
-  const long kt = cdiv(k, kFBK);
   const BalancedPlan b = balanced_plan(m, n, k, workers);
+  auto time = [&](int tile, int s) {
+    const float epi = s > 1 || store ? kEpiF32 : kEpiF32Add;
+    return tile_time(tile, m, n, k, kMNContig, kMNContig, workers, false, epi, s) +
+           (s > 1 ? reduce_time(m, n, s, store) : 0.0f);
+  };
   WgradPlan best{kTile256, splits, 0.0f};
-  if (splits <= 1 || b.sk_tiles == 0)
-    best.time = tile_time(kTile256, m, n, kt, kMNContig, kMNContig, workers);
-  else if (b.dp_tiles > 0)
-    best.time = balanced_time(b, workers);
+  if (splits > 1 && b.sk_tiles > 0 && b.dp_tiles > 0)
+    best.time = balanced_time(b, store, workers);
   else
-    best.time = tile_time(kTile256, m, n, cdiv(kt, splits), kMNContig, kMNContig, workers, splits) +
-                reduce_time(m, n, splits, store);
-  float limit = 0.88f * best.time;
+    best.time = time(kTile256, b.sk_tiles == 0 ? 1 : splits);
+  float limit = 0.9f * best.time;
   for (int tile = kTile256 + 1; tile < kFastTiles; ++tile)
     for (int s = 1; s <= splits; ++s) {
-      const float t = tile_time(tile, m, n, cdiv(kt, s), kMNContig, kMNContig, workers, s) +
-                      (s > 1 ? reduce_time(m, n, s, store) : 0.0f);
+      const float t = time(tile, s);
       if (t < limit) {
         best = WgradPlan{tile, s, t};
         limit = t;
@@ -489,7 +490,7 @@ int mm_f32_group(const ws_accumulate_problem* problems, int count, int64_t k, in
       apart += wgrad_plan(m, n, k, workspace ? auto_splits(m, n, k, workers) : 1,
                           (acc & kAccStore) != 0, workers).time;
     }
-    one_launch = apart >= 0.88f * balanced_time(plan, workers);
+    one_launch = apart >= 0.9f * balanced_time(plan, (acc & kAccStore) != 0, workers);
   }
   if (!one_launch) {
     for (int i = 0; i < count; ++i) {

@@ -102,12 +102,14 @@ struct GemmParams {
 
 // Spread a dispatch-order index so that the workgroups that run on one XCD at the same
 // time (the hardware deals workgroups round-robin to the 8 XCDs) get consecutive tiles.
+// XCD x of a window of 8 q + r workgroups has q + 1 of them when x < r and q otherwise. (Left
+// in launch order when r != 0, a 9000 x 7680 x 1536 product on 128 x 128 tiles took 282 us
+// instead of 211: the XCDs' L2 caches shared nothing.)
 __device__ __forceinline__ int xcd_remap(int w, int total, int window) {
-  int base = (w / window) * window;
-  int size = min(window, total - base);
-  if (size % kXcds != 0) return w;
-  int within = w - base;
-  return base + (within % kXcds) * (size / kXcds) + within / kXcds;
+  const int base = (w / window) * window;
+  const int size = min(window, total - base), q = size / kXcds, r = size % kXcds;
+  const int within = w - base, x = within % kXcds;
+  return base + x * q + min(x, r) + within / kXcds;
 }
 
 // Stream-K shares: worker v of W owns units [sk_begin(v), sk_begin(v + 1)) of U.

@@ -187,73 +187,104 @@ typedef RingCfg<64, 128, 2, 2, 3> Ring64x128;
 typedef RingCfg<64, 64, 2, 2, 4> Ring64;
 enum FastTile { kTile256 = 0, kTile128x2, kTile128x1, kTile64x128, kTile64, kFastTiles };
 
-// Cost of one launch of each macro-tile in microseconds, from a sweep of 32 shapes (128 to
-// 16384 rows, 512 to 32768 columns, K 512 to 16384; outputs of all tiles the same bits):
-// a CU runs its workgroups one after another (or two at a time), each taking `alone` us per
-// 64-deep k-tile, `pair` us for two that share the CU, and `fixed` us around its k-loop.
-// The 256 x 256 tile costs less per product with every CU busy; below about one round of
-// its tiles most CUs idle, and a smaller tile wins although it loads its operands more
-// often. Measured, us (256 x 256 against the choice): 512 x 1280 x 8960 159 / 40 (64 x 64),
-// 1999 x 1280 x 8960 158 / 71 (128 x 128 alone), 4096 x 1280 x 6400 114 / 71 (128 x 128
-// paired), 128 x 4800 x 960 23 / 7.4 (64 x 64); and where it stays: 8192 x 10240 x 2048
-// 250 / 294, 8192 x 2048 x 2048 54 / 59 (the best smaller tile).
+// Cost of one launch of each macro-tile in microseconds, fitted to sweeps of 150 shapes and
+// epilogues (128 to 16384 rows, 512 to 32768 columns, K 512 to 16384; outputs of all tiles the
+// same bits; the picks are within 2 % of the best tile in the geometric mean). A CU runs its
+// workgroups in rounds of one (`pair` 0) or two at a time; a round takes `alone` us per
+// 64-deep k-tile for one workgroup, `pair` us for two that share the CU, and `fixed` us
+// around the k-loop. The 256 x 256 tile costs less per product with every CU busy; below about
+// one round of its tiles most CUs idle, and a smaller tile wins although it loads its operands
+// more often. Measured, us (256 x 256 against the choice): 512 x 1280 x 8960 159 / 40
+// (64 x 64), 1999 x 1280 x 8960 158 / 71 (128 x 128 alone), 4096 x 1280 x 6400 114 / 71
+// (128 x 128 paired), 128 x 4800 x 960 23 / 7.4 (64 x 64); and where it stays: 8192 x 10240 x
+// 2048 250 / 294, 8192 x 2048 x 2048 54 / 59 (the best smaller tile).
 struct TileCost {
   int bm, bn;
   float alone, pair, fixed;  // pair 0: one workgroup per CU
+  // Over several rounds of pairs the workgroups drift apart and share less in L2: `pair`
+  // starts `settle` lower and grows by `drift` per k-tile beyond 32, to `most` at the end.
+  float settle, drift, most;
+  // Rows off whole 128-byte lines: the k-loop's factor when the contiguous reduction is no
+  // multiple of 64 (each row piece spans two lines), and us per round for such outputs.
+  float ragged_k, ragged_n;
 };
 inline const TileCost& tile_cost(int tile, int am, int bm) {
-  static const TileCost kk[kFastTiles] = {{256, 256, 1.55f, 0.0f, 4.0f},
-                                          {128, 128, 0.62f, 0.93f, 3.2f},
-                                          {128, 128, 0.50f, 0.0f, 3.6f},
-                                          {64, 128, 0.34f, 0.55f, 3.6f},
-                                          {64, 64, 0.28f, 0.36f, 3.4f}};
-  static const TileCost kmn[kFastTiles] = {{256, 256, 1.87f, 0.0f, 4.0f},
-                                           {128, 128, 0.64f, 0.95f, 3.2f},
-                                           {128, 128, 0.53f, 0.0f, 3.6f},
-                                           {64, 128, 0.38f, 0.58f, 3.6f},
-                                           {64, 64, 0.31f, 0.38f, 3.4f}};
-  static const TileCost mnmn[kFastTiles] = {{256, 256, 1.85f, 0.0f, 4.0f},
-                                            {128, 128, 0.60f, 1.00f, 3.2f},
-                                            {128, 128, 0.54f, 0.0f, 3.6f},
-                                            {64, 128, 0.39f, 0.70f, 3.6f},
-                                            {64, 64, 0.29f, 0.42f, 3.4f}};
+  static const TileCost kk[kFastTiles] = {
+      {256, 256, 1.55f, 0.0f, 4.0f, 0, 0, 0, 1.05f, 5.0f},
+      {128, 128, 0.62f, 0.87f, 3.2f, 0.07f, 0.006f, 0.18f, 1.25f, 5.0f},
+      {128, 128, 0.50f, 0.0f, 3.6f, 0, 0, 0, 1.1f, 1.7f},
+      {64, 128, 0.34f, 0.50f, 3.6f, 0.0f, 0.005f, 0.16f, 1.2f, 1.0f},
+      {64, 64, 0.28f, 0.33f, 3.4f, 0.0f, 0.0015f, 0.09f, 1.4f, 0.5f}};
+  static const TileCost kmn[kFastTiles] = {
+      {256, 256, 1.87f, 0.0f, 4.0f, 0, 0, 0, 1.05f, 5.0f},
+      {128, 128, 0.64f, 0.89f, 3.2f, 0.07f, 0.006f, 0.18f, 1.25f, 5.0f},
+      {128, 128, 0.53f, 0.0f, 3.6f, 0, 0, 0, 1.1f, 1.7f},
+      {64, 128, 0.38f, 0.53f, 3.6f, 0.0f, 0.005f, 0.16f, 1.2f, 1.0f},
+      {64, 64, 0.31f, 0.36f, 3.4f, 0.0f, 0.0015f, 0.09f, 1.4f, 0.5f}};
+  static const TileCost mnmn[kFastTiles] = {
+      {256, 256, 1.85f, 0.0f, 4.0f, 0, 0, 0, 1.0f, 5.0f},
+      {128, 128, 0.60f, 1.00f, 3.2f, 0, 0, 0, 1.0f, 5.0f},
+      {128, 128, 0.54f, 0.0f, 3.6f, 0, 0, 0, 1.0f, 1.7f},
+      {64, 128, 0.39f, 0.70f, 3.6f, 0, 0, 0, 1.0f, 1.0f},
+      {64, 64, 0.29f, 0.42f, 3.4f, 0, 0, 0, 1.0f, 0.5f}};
   if (am == kKContig && bm == kKContig) return kk[tile];
   return (am == kMNContig && bm == kMNContig ? mnmn : kmn)[tile];
 }
-// An [m, n] output (n the packed width of a paired GEMM) over k_tiles k-tiles, or `copies` of
-// it (split-K slices of k_tiles each).
-inline float tile_time(int tile, long m, long n, long k_tiles, int am, int bm, int cus,
-                       long copies = 1) {
+// What an epilogue costs beside a plain BF16 store, us per round of 256 x 256 tiles (every CU
+// in it at once, bound by HBM): the SwiGLU backward reads and writes the packed projection,
+// 8192 x 4096 x 1024 102 us against 58. A smaller tile's round pays by its area; two
+// workgroups on a CU hide a tenth of it behind each other's k-loop.
+enum EpiCost { kEpiStore = 0, kEpiSigmoid = 2, kEpiSwiglu = 4, kEpiF32 = 6, kEpiF32Add = 18, kEpiSwigluBwd = 20 };
+
+// An [m, n] output (n the packed width of a paired GEMM) with reduction k in `copies` split-K
+// slices.
+inline float tile_time(int tile, long m, long n, long k, int am, int bm, int cus, bool paired,
+                       float epi, long copies = 1) {
   const TileCost& c = tile_cost(tile, am, bm);
-  const long tiles = (long)cdiv(m, c.bm) * cdiv(n, c.bn) * copies, rounds = tiles / cus;
-  const float kt = (float)k_tiles;
-  if (tile == kTile256) {
+  const long tiles = (long)cdiv(m, c.bm) * cdiv(n, c.bn) * copies;
+  const float kt = (float)cdiv(cdiv(k, kFBK), copies), area = (float)(c.bm * c.bn) / 65536.0f;
+  const float slow = k % kFBK ? c.ragged_k : 1.0f;
+  const float fixed = c.fixed + ((paired ? n / 2 : n) % kFBK ? c.ragged_n : 0.0f);
+  const float alone = c.alone * slow;
+  if (c.pair == 0.0f) {
+    const long rounds = tiles / cus, rest = tiles % cus;
+    if (tile != kTile256) return (float)(rounds + (rest != 0)) * (alone * kt + fixed + epi * area);
     // With most CUs idle in the last round its tiles' loads meet less traffic.
-    float t = (float)rounds * (c.alone * kt + c.fixed);
-    if (tiles % cus) t += c.alone * (0.73f + 0.27f * (float)(tiles % cus) / (float)cus) * kt + c.fixed;
+    float t = (float)rounds * (alone * kt + fixed + epi);
+    if (rest) t += alone * (0.73f + 0.27f * (float)rest / (float)cus) * kt + fixed + epi;
     return t;
   }
-  const long per_cu = rounds + (tiles % cus != 0);
-  if (c.pair == 0.0f) return (float)per_cu * (c.alone * kt + c.fixed);
-  return (float)(per_cu / 2) * (c.pair * kt + c.fixed) + (float)(per_cu % 2) * (c.alone * kt + c.fixed);
+  const long rounds = tiles / (2 * cus), rest = tiles % (2 * cus);
+  const float around = fixed + epi * area * 1.8f;
+  float pair = c.pair * slow;
+  float drift = 0.0f;
+  if (tiles > 2 * cus) {
+    drift = -c.settle + c.drift * (kt - 32.0f);
+    drift = drift < -c.settle ? -c.settle : drift > c.most ? c.most : drift;
+  }
+  float t = (float)rounds * ((pair + drift) * kt + around);
+  if (rest > cus)  // some CUs hold a pair
+    t += (alone + (pair - alone) * (float)(rest - cus) / (float)cus) * kt + around;
+  else if (rest)
+    t += alone * kt + fixed + epi * area;
+  return t;
 }
-// The macro-tile with the lowest cost. A smaller one must promise 12 % over 256 x 256: with
-// several rounds of pairs on long reductions the estimates are up to that much too low
-// (8192 x 2048 x 10240: 304 estimated, 344 measured, 247 on 256 x 256).
-inline int pick_tile(long m, long n, long k, int am, int bm, bool paired, float* time = nullptr) {
+// The macro-tile with the lowest cost; a smaller one must promise 5 % over 256 x 256.
+inline int pick_tile(long m, long n, long k, int am, int bm, bool paired, float epi,
+                     float* time = nullptr) {
   const int cus = device_cus();
-  const long kt = cdiv(k, kFBK);
   int best = kTile256;
-  float t = 0.88f * tile_time(kTile256, m, n, kt, am, bm, cus);
+  const float whole = tile_time(kTile256, m, n, k, am, bm, cus, paired, epi);
+  float t = 0.95f * whole;
   // A paired 64 x 64 tile would write 32-byte row pieces.
   for (int i = 1; i < (paired ? kTile64 : kFastTiles); ++i) {
-    const float ti = tile_time(i, m, n, kt, am, bm, cus);
+    const float ti = tile_time(i, m, n, k, am, bm, cus, paired, epi);
     if (ti < t) {
       best = i;
       t = ti;
     }
   }
-  if (time) *time = best == kTile256 ? t / 0.88f : t;
+  if (time) *time = best == kTile256 ? whole : t;
   return best;
 }
 
@@ -287,8 +318,9 @@ int run_ring_tile(const GemmParams& p, int tile, hipStream_t s, int splits = 1) 
 constexpr unsigned kMaskKRows = ab_bit(kKContig, kKContig) | ab_bit(kKContig, kMNContig);
 constexpr unsigned kMaskVector = kMaskKRows | ab_bit(kMNContig, kKContig) | ab_bit(kMNContig, kMNContig);
 template <unsigned MASK, bool PAIRED, class Epi>
-int dispatch_tiles(const GemmParams& p, int am, int bm, LaunchCfg cfg, hipStream_t s) {
-  const int tile = (MASK & ab_bit(am, bm)) ? pick_tile(p.M, p.N, p.K, am, bm, PAIRED) : kTile256;
+int dispatch_tiles(const GemmParams& p, int am, int bm, LaunchCfg cfg, hipStream_t s,
+                   float epi = kEpiStore) {
+  const int tile = (MASK & ab_bit(am, bm)) ? pick_tile(p.M, p.N, p.K, am, bm, PAIRED, epi) : kTile256;
   if (tile == kTile256) return dispatch_fast<PAIRED, Epi>(p, am, bm, cfg, s);
 #define WS_RING(A_, B_)                                                          \
   if constexpr ((MASK & ab_bit(A_, B_)) != 0)                                    \

@@ -86,7 +86,7 @@ def k_contiguous_b(b: torch.Tensor, rows_a: int) -> torch.Tensor:
     return b
 
 
-def gemm_b(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+def gemm_b(a: torch.Tensor, b: torch.Tensor, swiglu_backward: bool = False) -> torch.Tensor:
     """B [K, N] as the GEMM of ``a`` [M, K] best reads it: ``k_contiguous_b``'s copy, or B
     itself where the vector loaders read an N-contiguous B directly at no loss: beside a
     token-major A (a weight gradient's dY.T: both operands go through the same transposing
@@ -97,7 +97,8 @@ def gemm_b(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     if b.stride(1) == 1 and n % 8 == 0 and b.stride(0) % 8 == 0 and b.data_ptr() % 16 == 0:
         token_major = (a.stride(0) == 1 and a.shape[0] % 8 == 0 and a.stride(1) % 8 == 0
                        and a.data_ptr() % 16 == 0)
-        if token_major or not _hip.query("ws_mm_copy_pays", a.shape[0], n, k):
+        if token_major or not _hip.query("ws_mm_copy_pays", a.shape[0], n, k,
+                                         int(swiglu_backward)):
             return b
     return k_contiguous_b(b, a.shape[0])
 
@@ -248,7 +249,10 @@ def swiglu_backward_mm(grad: torch.Tensor, down_weight: torch.Tensor, packed: to
     if out is None:
         out = torch.empty((m, 2 * h), dtype=torch.bfloat16, device=grad.device)
     _check_buffer(out, (m, 2 * h), torch.bfloat16, grad.device, "out")
-    down_weight = gemm_b(grad, down_weight)
+    # From 16384 rows the 256 x 256 tiles on a copy and the paired 128 x 128 ones on the weight
+    # itself are level (h 5632, d 2048: 401-425 + 14 us against 421); below, the copy loses.
+    down_weight = (k_contiguous_b(down_weight, m) if m >= 16384
+                   else gemm_b(grad, down_weight, True))
     _hip.call("ws_swiglu_backward_mm", grad.data_ptr(), grad.stride(0), grad.stride(1),
               down_weight.data_ptr(), down_weight.stride(0), down_weight.stride(1),
               packed.data_ptr(), out.data_ptr(), m, h, k, int(eager_rounding), _hip.stream(grad))
