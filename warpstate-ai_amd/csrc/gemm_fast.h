@@ -657,7 +657,10 @@ struct FEpiCEGrad {
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's staging writes landed
     const int c8 = 8 * (lane & 15);
     const int n = n_base + c8;
-    const bool full = n + 7 < p.N, half = n + 3 < p.N;  // N % 4 == 0 (vec_out)
+    // Rows are ldc long: N, a multiple of 4, or padded past a ragged N with zero gradients.
+    const int n_out = (int)p.ldc;
+    const bool full = n + 7 < n_out, half = n + 3 < n_out;
+    const bool padded = n_out > p.N && n_base + FB * 16 > p.N;  // wave-uniform
     __amdgpu_buffer_rsrc_t rc = make_rsrc(p.c + (long)m_base * p.ldc + n_base, 0x7fffffff);
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
@@ -685,6 +688,11 @@ struct FEpiCEGrad {
         for (int d = 0; d < 4; ++d)
           o[d] = pack_bf16x2(scale * exp_e(lo_bf16(vl[d]) - lse), scale * exp_e(hi_bf16(vl[d]) - lse));
       }
+      if (padded) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          o[d] &= (n + 2 * d < p.N ? 0xffffu : 0u) | (n + 2 * d + 1 < p.N ? 0xffff0000u : 0u);
+      }
       const long off = (long)r * p.ldc + c8;
       if (full) {
         __builtin_amdgcn_raw_buffer_store_b128(o, rc, store_off(ok, off, 2), 0, kEpiNT);
@@ -696,8 +704,8 @@ struct FEpiCEGrad {
 };
 
 // LM-head pass 1 that also keeps the logits: the statistics of FEpiCEStats, then the
-// rounded BF16 logits through the wave's LDS staging rows into c [M, N] (row stride ldc,
-// N % 4 == 0) as 16-byte row pieces, so that the backward reads them instead of
+// rounded BF16 logits through the wave's LDS staging rows into c [M, ldc] (ldc = N, a
+// multiple of 4, or N padded to a multiple of 64) as 16-byte row pieces, so that the backward reads them instead of
 // recomputing the GEMM.
 struct FEpiCEStatsLogits {
   template <int FA, int FB>
@@ -720,7 +728,10 @@ struct FEpiCEStatsLogits {
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's staging writes landed
     const int c8 = 8 * (lane & 15);
     const int n = n_base + c8;
-    const bool full = n + 7 < p.N, half = n + 3 < p.N;
+    // Rows are ldc long: N, a multiple of 4, or padded past a ragged N (with the -inf that the
+    // statistics put there, whose logit gradients are zero).
+    const int n_out = (int)p.ldc;
+    const bool full = n + 7 < n_out, half = n + 3 < n_out;
     __amdgpu_buffer_rsrc_t rc = make_rsrc(p.c + (long)m_base * p.ldc + n_base, 0x7fffffff);
 #pragma unroll
     for (int q = 0; q < 16; ++q) {

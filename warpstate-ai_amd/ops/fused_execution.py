@@ -455,6 +455,14 @@ def _check_state(state: CrossEntropyState, rows: int, vocab: int, device) -> Non
         raise ValueError("CrossEntropyState chunk_rows must lie in [1, rows]")
 
 
+def _head_weight_t(weight: torch.Tensor, rows: int) -> torch.Tensor | None:
+    """The head weight transposed for the dHidden GEMM (K-contiguous B) when there are enough
+    rows to amortize the copy, which has 16-byte rows only for a vocabulary that is a multiple
+    of 8."""
+    return (transpose(weight) if rows >= TRANSPOSE_MIN_ROWS and weight.shape[0] % 8 == 0
+            else None)
+
+
 def linear_cross_entropy_forward(hidden: torch.Tensor, weight: torch.Tensor,
                                  targets: torch.Tensor, state: CrossEntropyState | None = None
                                  ) -> CrossEntropyState:
@@ -470,7 +478,7 @@ def linear_cross_entropy_forward(hidden: torch.Tensor, weight: torch.Tensor,
         if state.d != d:
             raise ValueError(f"The fused CrossEntropyState was built for d={state.d}, not {d}")
         workspace = state.backward_workspace(d)
-        weight_t = transpose(weight) if rows >= TRANSPOSE_MIN_ROWS else None
+        weight_t = _head_weight_t(weight, rows)
         # Kept for the backward's two-pass fallback (an upstream gradient that is not a
         # power of two).
         state.weight_t = weight_t
@@ -535,7 +543,7 @@ def linear_cross_entropy_backward(hidden: torch.Tensor, weight: torch.Tensor,
         return out
     workspace = state.backward_workspace(d)
     # The dHidden GEMM reads the head weight along the vocabulary: give it W^T rows.
-    weight_t = transpose(weight) if rows >= TRANSPOSE_MIN_ROWS else None
+    weight_t = _head_weight_t(weight, rows)
     _hip.call("ws_linear_ce_backward", hidden.data_ptr(), hidden.stride(0), weight.data_ptr(),
               weight.stride(0), None if weight_t is None else weight_t.data_ptr(),
               targets.data_ptr(), state.lse.data_ptr(), state.count.data_ptr(),
