@@ -54,13 +54,6 @@ const char* ws_version(void);
 int ws_mm(const void* a, int64_t a_s0, int64_t a_s1, const void* b, int64_t b_s0, int64_t b_s1,
           void* c, int64_t m, int64_t n, int64_t k, int algorithm, int tile, void* stream);
 
-/* Whether a product A[m,k] @ B[k,n] of a K-contiguous A and an N-contiguous B is expected to
- * run faster on a K-contiguous copy of B (ws_transpose_bf16), the copy's time included: 1 or
- * 0. A host-side rule on the sizes (and the current device's compute units), for a plain
- * store or, with swiglu_backward, ws_swiglu_backward_mm's epilogue; the product is the same
- * either way. */
-int ws_mm_copy_pays(int64_t m, int64_t n, int64_t k, int swiglu_backward);
-
 /*
  * Paired up/gate projection with SwiGLU epilogue: packed[m, 2h] = bf16(A @ B) (up in
  * columns [0,h), gate in [h,2h)), act[m,h] = bf16(r?(silu(gate)) * up), where silu runs

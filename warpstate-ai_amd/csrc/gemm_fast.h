@@ -6,7 +6,7 @@
 // in input gradients are M/N-contiguous).
 //
 // Workgroup: 256 x 256 output tile, BK = 64, 8 waves on a 4 x 2 grid (wave tile 64 x 128),
-// two LDS stages of 64 KiB (A 32 KiB + B 32 KiB).
+// A in two LDS stages and B in three (160 KiB).
 //  * Loads: `buffer_load_dword x4 ... lds` writes 16 bytes per lane straight into LDS at
 //    M0 + 16 * lane; the choice of global address per lane implements the LDS swizzle.
 //    Out-of-range rows, columns and k take an offset beyond the buffer's range and land
@@ -26,22 +26,21 @@
 //  * MFMA v_mfma_f32_16x16x32_bf16 with the B fragment as the instruction's A operand:
 //    lane l then holds output row m = m0 + 16 i + (l & 15), columns n0 + 16 j + 4 (l >> 4)
 //    + e, e = 0..3, which the epilogues store as 8-byte (BF16) or 16-byte (FP32) vectors.
-//  * Pipeline per k-tile, both operands K-contiguous: A has two LDS stages and B three
-//    (160 KiB). Wait for this wave's loads of the tile (leaving the 4 loads of B two tiles
-//    ahead in flight), s_barrier (no memory fence: the explicit vmcnt wait is the only
-//    ordering needed), issue A of the next tile, then the two k32 steps with the second
-//    step's fragment reads interleaved between the first step's MFMAs, and between the two
-//    steps the loads of B two tiles ahead. Those land while the second step runs without
-//    LDS reads, and only half a tile's loads leave in a burst after the barrier (the
-//    forward GEMMs 3-7 % faster than with both operands' next tile loaded there).
-//  * Both operands M/N-contiguous (the weight gradients): two stages of 64 KiB; after the
-//    barrier the next tile's loads for both operands, then the transposing fragment reads.
-//    The reads are inline assembly with explicit lgkmcnt waits: the compiler orders the
-//    transposing-read builtin after every pending direct-to-LDS load (it cannot rule out
-//    an alias), which would otherwise hold those loads back until after the tile's last
-//    read and leave them half a k-tile of lead (the weight gradients 9 % slower).
-//  * One operand of each kind: both in two stages, the next tile's loads between the two
-//    steps (after the tile's last transposing read).
+//  * Pipeline: the waves form two groups, 0-3 and 4-7, one wave of each on every SIMD, that
+//    run one phase apart. A k-tile takes a group two phases with a barrier after each: a read
+//    phase (its loads for a later k-tile, then all 24 fragments of this one) and an MFMA phase
+//    (64 MFMAs with nothing to wait for), so that on every SIMD one wave's MFMAs run while
+//    the other's fragments and loads move. The first group loads A one k-tile ahead (two
+//    phases), the second B two ahead (three phases); a stage is refilled only after both
+//    groups have read it. The 8 waves in step on one barrier per k-tile left the matrix pipe
+//    idle while all of them read their first fragments; one box, alternated, same bits, us:
+//    16384 x 9216 x 2048 460 -> 436, 16384 x 2048 x 11264 536 -> 501, 8192 x 8192 x 8192
+//    772 -> 717 (1.53 PFLOP/s), 16384 x 2048 x 5632 275 -> 257. Moving B's second-step reads
+//    into the MFMA phase, s_setprio around it and the loads between the reads change nothing:
+//    the clock gives way (32x32x16 MFMAs: 11 % slower).
+//  * The fragment reads are inline assembly with explicit lgkmcnt waits: the compiler orders
+//    the transposing-read builtin after every pending direct-to-LDS load (it cannot rule out
+//    an alias), which would wait for the loads of the tile ahead.
 //  * Tiles follow the grouped raster of ops/matmul_kernels.py:72-78 after an XCD remap.
 #pragma once
 
@@ -54,21 +53,16 @@ namespace ws {
 constexpr int kFBM = 256, kFBN = 256, kFBK = 64, kFWM = 4, kFWN = 2;
 constexpr int kFNT = kFWM * kFWN * kWave;               // 512 threads
 constexpr int kFTileBytes = 256 * kFBK * 2;             // one operand tile, 32 KiB
-constexpr int kFStageBytes = 2 * kFTileBytes;
-constexpr int kFLdsBytes = 2 * kFStageBytes;            // 128 KiB
+// A in two LDS stages, B in three: the whole 160 KiB of a CU.
+constexpr int kFLdsBytes = 5 * kFTileBytes;
 // Epilogue staging: each wave's BF16 tile of FA x FB blocks (64 x 128 here), rows padded by
 // 16 bytes (to 272) so that both the fragment-order writes and the row-order 16-byte reads
 // are bank-conflict free.
 template <int FB> constexpr int epi_row() { return FB * 32 + 16; }
 template <int FA, int FB> constexpr int epi_wave() { return FA * 16 * epi_row<FB>(); }
 constexpr int kFStageWave = epi_wave<4, 8>();
-constexpr int kFLdsAlloc = 8 * kFStageWave > kFLdsBytes ? 8 * kFStageWave : kFLdsBytes;
-// Both operands K-contiguous: A in two stages, B in three (the whole 160 KiB of a CU).
-constexpr int kFLdsAllocKK = 5 * kFTileBytes;
-static_assert(kFLdsAllocKK >= 8 * kFStageWave, "the epilogue staging fits the K-contiguous layout");
-template <int AM, int BM>
-constexpr int fast_lds_bytes() { return AM == kKContig && BM == kKContig ? kFLdsAllocKK : kFLdsAlloc; }
-constexpr int kFIns = kFTileBytes / (kFNT * 16);         // 4 loads per thread per operand
+static_assert(kFLdsBytes >= 8 * kFStageWave, "the epilogue staging fits the operand stages");
+constexpr int kFIns = kFTileBytes / (kFNT / 2 * 16);     // 8 loads per thread of its group's operand
 // Cache policy of the epilogues' outputs and auxiliary inputs: non-temporal. Each is
 // touched once, in bursts when all CUs reach their epilogues together, and it should not
 // displace the operand tiles that other workgroups are still reading from L2 (dAct 4-5 %
@@ -86,55 +80,50 @@ constexpr int wait_vmcnt(int n) { return (n & 0xF) | (7 << 4) | (0xF << 8) | ((n
 
 #define WS_LDS(p) ((__attribute__((address_space(3))) void*)(p))
 
-// Direct-to-LDS loader of one 256-row operand tile. `off[i]` is the byte offset of this
-// lane's 16-byte chunk for load i relative to the tile's global base at k0, or kOOB.
-template <int MODE, bool PAIRED>
-struct DmaTile {
-  unsigned off[kFIns];
+// 16 bytes per lane from `rs` at byte offset `off` into LDS at lds + 16 * lane. (A function
+// of its own: with template-dependent arguments the builtin's target check fails on the
+// compiler's host pass.)
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, unsigned char* lds, unsigned off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, WS_LDS(lds), 16, off, 0, 0, 0);
+}
 
-  // k offset within the tile of load i's chunk: 8 c (K-contiguous) or the k-row kk.
+// Direct-to-LDS loader of a ROWS x 64 operand tile by NT threads, in the tile layouts of
+// the header comment (K-contiguous: [ROWS][64 k] with swizzled 16-byte chunks; M/N-contiguous:
+// blocks of 64 operand rows, each [64 k][128 B]).
+template <int ROWS, int NT, int MODE, bool PAIRED>
+struct RingTile {
+  static constexpr int kIns = ROWS * 8 / NT;
+  static_assert(kIns >= 1 && ROWS * 8 % NT == 0 && ROWS % 64 == 0, "whole loads per thread");
+  unsigned off[kIns];
+
   __device__ __forceinline__ static int k_of(int i, int wave, int lane) {
-    const int byte = (i * (kFNT / kWave) + wave) * 1024 + lane * 16;
+    const int byte = (i * (NT / kWave) + wave) * 1024 + lane * 16;
     if constexpr (MODE == kKContig) return 8 * (((byte >> 4) & 7) ^ swz(byte >> 7));
     else return ((byte >> 10) & 7) * 8 + (lane >> 3);
   }
   __device__ __forceinline__ void init(const OperandDesc& d, int row0, int rows_valid, int half,
                                        int wave, int lane) {
 #pragma unroll
-    for (int i = 0; i < kFIns; ++i) {
-      const int byte = (i * (kFNT / kWave) + wave) * 1024 + lane * 16;
+    for (int i = 0; i < kIns; ++i) {
+      const int byte = (i * (NT / kWave) + wave) * 1024 + lane * 16;
+      int r, c = 0, kk = 0;
       if constexpr (MODE == kKContig) {
-        const int r = byte >> 7, c = ((byte >> 4) & 7) ^ swz(r);
-        const int logical = row0 + (PAIRED && r >= 128 ? r - 128 : r);
-        const int phys = PAIRED && r >= 128 ? half + logical : logical;
-        off[i] = logical < rows_valid ? (unsigned)((long)(phys - row0) * d.s_row * 2 + 16 * c) : kOOB;
+        r = byte >> 7;
+        c = ((byte >> 4) & 7) ^ swz(r);
       } else {
-        const int q = byte >> 10, kk = (q & 7) * 8 + (lane >> 3);
-        const int c = (lane & 7) ^ mnsw(kk);
-        const int r = (q >> 3) * 64 + 8 * c;  // first operand row of the chunk
-        const int logical = row0 + (PAIRED && r >= 128 ? r - 128 : r);
-        const int phys = PAIRED && r >= 128 ? half + logical : logical;
-        off[i] = logical < rows_valid ? (unsigned)((phys - row0) * 2 + (long)kk * d.s_k * 2) : kOOB;
+        const int q = byte >> 10;
+        kk = (q & 7) * 8 + (lane >> 3);
+        r = (q >> 3) * 64 + 8 * ((lane & 7) ^ mnsw(kk));  // first operand row of the chunk
       }
+      const int logical = row0 + (PAIRED && r >= ROWS / 2 ? r - ROWS / 2 : r);
+      const int phys = PAIRED && r >= ROWS / 2 ? half + logical : logical;
+      const long rel = MODE == kKContig ? (long)(phys - row0) * d.s_row * 2 + 16 * c
+                                        : (phys - row0) * 2 + (long)kk * d.s_k * 2;
+      off[i] = logical < rows_valid ? (unsigned)rel : kOOB;
     }
   }
-  // Load i alone of the tile at k0, branch-free so that it can be scheduled among MFMAs:
-  // a chunk at k >= K, or every chunk when `live` is false, takes the out-of-range offset
-  // and lands as zeros without a memory read.
-  __device__ __forceinline__ void issue_one(const OperandDesc& d, int row0, int k0, int K,
-                                            unsigned char* lds_tile, int wave, int lane, int i,
-                                            bool live) const {
-    const unsigned short* base =
-        MODE == kKContig ? d.ptr + (long)row0 * d.s_row + k0 : d.ptr + row0 + (long)k0 * d.s_k;
-    __amdgpu_buffer_rsrc_t rs = make_rsrc(base, 0x7fffffff);
-    int l = lane;
-    asm volatile("" : "+v"(l));
-    const bool dead = !live | (k0 + k_of(i, wave, l) >= K);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, WS_LDS(lds_tile + (i * (kFNT / kWave) + wave) * 1024),
-                                             16, dead ? kOOB : off[i], 0, 0, 0);
-  }
-  // Loads of the tile at k0 into `lds_tile`; chunks at k >= K load zeros. The per-lane k
-  // test only runs on a ragged last tile.
+  // The tile at k0 into `lds_tile`; chunks at k >= K (all of them past the last k-tile)
+  // land as zeros, so that every wait counts the same number of loads.
   __device__ __forceinline__ void issue(const OperandDesc& d, int row0, int k0, int K,
                                         unsigned char* lds_tile, int wave, int lane) const {
     const unsigned short* base =
@@ -142,51 +131,29 @@ struct DmaTile {
     __amdgpu_buffer_rsrc_t rs = make_rsrc(base, 0x7fffffff);
     if (k0 + kFBK <= K) {
 #pragma unroll
-      for (int i = 0; i < kFIns; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, WS_LDS(lds_tile + (i * (kFNT / kWave) + wave) * 1024),
-                                                 16, off[i], 0, 0, 0);
+      for (int i = 0; i < kIns; ++i)
+        dma16(rs, lds_tile + (i * (NT / kWave) + wave) * 1024, off[i]);
     } else {
-      // Ragged last k-tile. The lane index goes through an empty asm so that the per-lane
-      // k offsets are computed here and not kept live across the k-loop.
       int l = lane;
       asm volatile("" : "+v"(l));
 #pragma unroll
-      for (int i = 0; i < kFIns; ++i) {
+      for (int i = 0; i < kIns; ++i) {
         const unsigned o = k0 + k_of(i, wave, l) >= K ? kOOB : off[i];
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, WS_LDS(lds_tile + (i * (kFNT / kWave) + wave) * 1024),
-                                                 16, o, 0, 0, 0);
+        dma16(rs, lds_tile + (i * (NT / kWave) + wave) * 1024, o);
       }
     }
   }
 };
 
-// Fragment reads for 16-row block at tile row `rb` (multiple of 16), k32 step s.
-template <int MODE>
+// Fragment read of a K-contiguous tile for the 16-row block at tile row `rb` (a multiple of
+// 16), k32 step s.
 __device__ __forceinline__ bf16x8_t read_frag(const unsigned char* tile, int rb, int s, int lane) {
-  if constexpr (MODE == kKContig) {
-    const int r = rb + (lane & 15);
-    const int c = (4 * s + (lane >> 4)) ^ swz(r);
-    return *reinterpret_cast<const bf16x8_t*>(tile + r * 128 + c * 16);
-  } else {
-    const int L = lane & 15, g = lane >> 4;
-    const int m = rb + 4 * (L & 3);
-    const int kk0 = 32 * s + 8 * g + (L >> 2);
-    const int kk1 = kk0 + 4;
-    const int blk = (m >> 6) * 8192, c = (m >> 3) & 7, hb = (m & 4) * 2;  // hb: 0 or 8
-    const unsigned char* p0 = tile + blk + kk0 * 128 + ((c ^ mnsw(kk0)) << 4) + hb;
-    const unsigned char* p1 = tile + blk + kk1 * 128 + ((c ^ mnsw(kk1)) << 4) + hb;
-    i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) i16x4_t*)(p0));
-    i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) i16x4_t*)(p1));
-    typedef short i16x8_t __attribute__((ext_vector_type(8)));
-    i16x8_t v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    return __builtin_bit_cast(bf16x8_t, v);
-  }
+  const int r = rb + (lane & 15);
+  const int c = (4 * s + (lane >> 4)) ^ swz(r);
+  return *reinterpret_cast<const bf16x8_t*>(tile + r * 128 + c * 16);
 }
 
-// Transposing fragment reads as inline assembly, for the loop with both operands
-// M/N-contiguous. The compiler does not see them as LDS accesses, so the direct-to-LDS
+// Transposing fragment reads as inline assembly. The compiler does not see them as LDS accesses, so the direct-to-LDS
 // loads of the next tile may be issued before them without an added vmcnt wait; their
 // results are made visible by tie_wait, an explicit lgkmcnt(0) that redefines the
 // fragment registers, so no MFMA reading them can be scheduled ahead of the wait.
@@ -197,16 +164,16 @@ __device__ __forceinline__ u32x2_t tr_read(unsigned addr) {
   return v;
 }
 // Fragment of k32 step S at LDS byte address `addr` (tr_base plus the stage offset): the
-// two reads of read_frag<kMNContig>, k-rows kk0 and kk0 + 4 (the same swizzle, 512 bytes
+// two reads are k-rows kk0 and kk0 + 4 (the same swizzle, 512 bytes
 // apart); step 1 is 32 k-rows (4096 bytes) further with the same swizzle.
-template <int S>
+template <int S, int OFF = 0>
 __device__ __forceinline__ bf16x8_t tr_frag(unsigned addr) {
-  const u32x2_t lo = tr_read<S * 4096>(addr), hi = tr_read<S * 4096 + 512>(addr);
+  const u32x2_t lo = tr_read<OFF + S * 4096>(addr), hi = tr_read<OFF + S * 4096 + 512>(addr);
   const u32x4_t v = {lo[0], lo[1], hi[0], hi[1]};
   return __builtin_bit_cast(bf16x8_t, v);
 }
 // Byte offset, within an M/N-contiguous operand tile, of lane's first read of the
-// fragment of the 16-row block at tile row rb, k32 step 0 (read_frag<kMNContig>).
+// fragment of the 16-row block at tile row rb, k32 step 0.
 __device__ __forceinline__ unsigned tr_base(int rb, int lane) {
   const int L = lane & 15, g = lane >> 4;
   const int m = rb + 4 * (L & 3);
@@ -214,10 +181,51 @@ __device__ __forceinline__ unsigned tr_base(int rb, int lane) {
   const int blk = (m >> 6) * 8192, c = (m >> 3) & 7, hb = (m & 4) * 2;
   return (unsigned)(blk + kk0 * 128 + ((c ^ mnsw(kk0)) << 4) + hb);
 }
-__device__ __forceinline__ void tie_wait(bf16x8_t (&f)[12]) {
+// One K-contiguous fragment read (read_frag) as inline assembly.
+template <int OFF>
+__device__ __forceinline__ bf16x8_t b128_read(unsigned addr) {
+  u32x4_t v;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "i"(OFF) : "memory");
+  return __builtin_bit_cast(bf16x8_t, v);
+}
+
+// LDS byte offset, within an operand tile, of this lane's piece of the fragment of the 16-row
+// block at tile row rb (a multiple of 64), k32 step 0.
+template <int MODE>
+__device__ __forceinline__ unsigned frag_base(int rb, int lane) {
+  if constexpr (MODE == kMNContig) return tr_base(rb, lane);
+  const int r = rb + (lane & 15);
+  return (unsigned)(r * 128 + (((lane >> 4) ^ swz(r)) << 4));
+}
+// Fragment of block J after the one at `base` (frag_base plus the stage), k32 step STEP. Rows of
+// K-contiguous blocks are 2048 bytes apart and step 1 is chunk c ^ 4; M/N-contiguous blocks
+// differ in bits 5 and 6 of the swizzled address within a 64-row block of 8 KiB. In a SPLIT
+// (paired) tile the blocks from J = 4 on lie 128 tile rows further.
+template <int MODE, int STEP, int J, bool SPLIT>
+__device__ __forceinline__ bf16x8_t asm_frag(unsigned base) {
+  if constexpr (MODE == kKContig)
+    return b128_read<SPLIT && J >= 4 ? 16384 + (J - 4) * 2048 : J * 2048>(base ^ (STEP * 64));
+  else
+    return tr_frag<STEP, (J >> 2) * (SPLIT ? 16384 : 8192)>(base ^ ((J & 3) * 32));
+}
+// Fragments I.. of both steps of a k-tile: per step 4 A blocks, then 8 B blocks.
+template <int AMODE, int BMODE, bool PAIRED, int I>
+__device__ __forceinline__ void asm_frags(bf16x8_t (&f)[24], unsigned a, unsigned b) {
+  if constexpr (I < 24) {
+    constexpr int step = I / 12, j = I % 12;
+    if constexpr (j < 4) f[I] = asm_frag<AMODE, step, j, false>(a);
+    else f[I] = asm_frag<BMODE, step, j - 4, PAIRED>(b);
+    asm_frags<AMODE, BMODE, PAIRED, I + 1>(f, a, b);
+  }
+}
+// Waits for every LDS read issued so far and redefines the fragment registers, so that no
+// MFMA that reads them can be scheduled ahead of the wait.
+__device__ __forceinline__ void tie_wait(bf16x8_t (&f)[24]) {
   asm volatile("s_waitcnt lgkmcnt(0)"
                : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]),
-                 "+v"(f[6]), "+v"(f[7]), "+v"(f[8]), "+v"(f[9]), "+v"(f[10]), "+v"(f[11])
+                 "+v"(f[6]), "+v"(f[7]), "+v"(f[8]), "+v"(f[9]), "+v"(f[10]), "+v"(f[11]),
+                 "+v"(f[12]), "+v"(f[13]), "+v"(f[14]), "+v"(f[15]), "+v"(f[16]), "+v"(f[17]),
+                 "+v"(f[18]), "+v"(f[19]), "+v"(f[20]), "+v"(f[21]), "+v"(f[22]), "+v"(f[23])
                :: "memory");
 }
 
@@ -756,17 +764,7 @@ __global__ void __launch_bounds__(kFNT) gemm_fast_kernel(const GemmParams p) {
   static_assert(AMODE != kGeneric && BMODE != kGeneric, "fast path needs vector operands");
   constexpr int TM = kFBM / kFWM, TN = kFBN / kFWN;  // 64 x 128
   constexpr int FA = TM / 16, FB = TN / 16;          // 4 x 8
-  constexpr int RA = AMODE == kKContig ? 1 : 2, RB = BMODE == kKContig ? 1 : 2;
-  constexpr int NR = FA * RA + FB * RB;              // DS read instructions per k32 step
-  constexpr int NM = FA * FB;                        // MFMAs per k32 step
-  // With an M/N-contiguous operand the next k-tile's loads are issued in the middle of
-  // the k-tile, after the last fragment read: their LDS writes then fall in the
-  // read-free second half instead of competing with the transposing reads (12-16 %
-  // faster). With both operands K-contiguous, A keeps the full k-tile of lead time
-  // (issuing it mid-tile costs 10 % there) and B, with a third stage, two k-tiles.
-  constexpr bool kMidIssue = AMODE == kMNContig || BMODE == kMNContig;
-  // Both operands M/N-contiguous (and not paired): the loop with assembly fragment reads.
-  constexpr bool kBothMN = AMODE == kMNContig && BMODE == kMNContig && !PAIRED;
+  static_assert(FA == 4 && FB == 8, "asm_frags reads 4 A and 8 B blocks per step");
 
   extern __shared__ __attribute__((aligned(1024))) unsigned char fsmem[];
   if (p.skip_if != nullptr && *p.skip_if != 0) return;  // uniform: the whole grid exits
@@ -774,21 +772,19 @@ __global__ void __launch_bounds__(kFNT) gemm_fast_kernel(const GemmParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / kFWN, wn = wave % kFWN;
+  const bool first = wave < 4;  // the group that runs a phase ahead and loads A
   const int bn_cols = PAIRED ? kFBN / 2 : kFBN;
   const int k_tiles_total = cdiv(p.K, kFBK);
   const int kt_begin = blockIdx.y * p.k_tiles_per_split;
   const int kt_end = min(k_tiles_total, kt_begin + p.k_tiles_per_split);
 
-  DmaTile<AMODE, false> la;
-  DmaTile<BMODE, PAIRED> lb;
-
-  // Tile rows of this wave's fragments (B rows for paired tiles: up blocks then gate).
-  int b_rb[FB];
-#pragma unroll
-  for (int j = 0; j < FB; ++j) {
-    if (PAIRED) b_rb[j] = (j < FB / 2) ? wn * (TN / 2) + 16 * j : 128 + wn * (TN / 2) + 16 * (j - FB / 2);
-    else b_rb[j] = wn * TN + 16 * j;
-  }
+  unsigned char* const sA = fsmem;                    // A stage c at sA + c * 32 KiB
+  unsigned char* const sB = fsmem + 2 * kFTileBytes;  // B stage c at sB + c * 32 KiB
+  const unsigned lds0 =
+      (unsigned)(unsigned long)(__attribute__((address_space(3))) unsigned char*)fsmem;
+  const unsigned abase = lds0 + frag_base<AMODE>(wm * TM, lane);
+  const unsigned bbase =
+      lds0 + 2 * kFTileBytes + frag_base<BMODE>(PAIRED ? wn * (TN / 2) : wn * TN, lane);
 
   // One output tile (raster index t of GEMM q) over k-tiles [kb, ke), then `epi(acc,
   // m_base, n_base, tm, tn)` and a barrier (the next tile's loads reuse the epilogue's
@@ -798,8 +794,6 @@ __global__ void __launch_bounds__(kFNT) gemm_fast_kernel(const GemmParams p) {
     tile_position(t, q.tiles_m, q.tiles_n, tm, tn);
     const int row0_a = tm * kFBM;
     const int row0_b = tn * bn_cols;
-    la.init(q.a, row0_a, q.M, 0, wave, lane);
-    lb.init(q.b, row0_b, PAIRED ? p.H : q.N, PAIRED ? p.H : 0, wave, lane);
 
     Acc16<FA, FB> acc;
 #pragma unroll
@@ -807,170 +801,94 @@ __global__ void __launch_bounds__(kFNT) gemm_fast_kernel(const GemmParams p) {
 #pragma unroll
       for (int j = 0; j < FB; ++j) acc.v[i][j] = f32x4_v{0.f, 0.f, 0.f, 0.f};
 
-    if (kb < ke && !kMidIssue) {
-      unsigned char* const sA = fsmem;                    // A stage c at sA + c * 32 KiB
-      unsigned char* const sB = fsmem + 2 * kFTileBytes;  // B stage c at sB + c * 32 KiB
-      la.issue(q.a, row0_a, kb * kFBK, p.K, sA, wave, lane);
-      lb.issue(q.b, row0_b, kb * kFBK, p.K, sB, wave, lane);
-      // B of the second k-tile, or zero-filling loads of the same count, so that every wait
-      // below leaves exactly the last kFIns loads (B two tiles ahead) in flight.
+    if (kb < ke) {
+      // This wave's share of its group's operand tile: one quarter, eight loads, at `base`
+      // plus `step` elements per k-tile.
+      typedef RingTile<256, 256, AMODE, false> TileA;
+      typedef RingTile<256, 256, BMODE, PAIRED> TileB;
+      const int gw = wave & 3;
+      unsigned off[kFIns];
+      const unsigned short* base;
+      long step;
+      if (first) {
+        TileA l;
+        l.init(q.a, row0_a, q.M, 0, gw, lane);
 #pragma unroll
-      for (int i = 0; i < kFIns; ++i)
-        lb.issue_one(q.b, row0_b, (kb + 1) * kFBK, p.K, sB + kFTileBytes, wave, lane, i, kb + 1 < ke);
-      int bst = 0;  // B stage of k-tile kt: (kt - kb) % 3
+        for (int i = 0; i < kFIns; ++i) off[i] = l.off[i];
+        base = q.a.ptr + (AMODE == kKContig ? row0_a * q.a.s_row : (long)row0_a);
+        step = AMODE == kKContig ? kFBK : kFBK * q.a.s_k;
+      } else {
+        TileB l;
+        l.init(q.b, row0_b, PAIRED ? p.H : q.N, PAIRED ? p.H : 0, gw, lane);
+#pragma unroll
+        for (int i = 0; i < kFIns; ++i) off[i] = l.off[i];
+        base = q.b.ptr + (BMODE == kKContig ? row0_b * q.b.s_row : (long)row0_b);
+        step = BMODE == kKContig ? kFBK : kFBK * q.b.s_k;
+      }
+      auto load = [&](int kt, unsigned char* stage) {
+        __amdgpu_buffer_rsrc_t rs = make_rsrc(base + kt * step, 0x7fffffff);
+        unsigned char* dst = stage + gw * 1024;
+        if ((kt + 1) * kFBK <= p.K) {
+#pragma unroll
+          for (int i = 0; i < kFIns; ++i) dma16(rs, dst + i * 4096, off[i]);
+        } else {
+          // Ragged or past the end: chunks at k >= K land as zeros. The lane index goes
+          // through an empty asm so that the k offsets are not kept live across the loop.
+          int l = lane;
+          asm volatile("" : "+v"(l));
+#pragma unroll
+          for (int i = 0; i < kFIns; ++i) {
+            const int k = first ? TileA::k_of(i, gw, l) : TileB::k_of(i, gw, l);
+            dma16(rs, dst + i * 4096, kt * kFBK + k >= p.K ? kOOB : off[i]);
+          }
+        }
+      };
+      if (first) {
+        load(kb, sA);
+        __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
+      } else {
+        load(kb, sB);
+        load(kb + 1, sB + kFTileBytes);
+        __builtin_amdgcn_s_waitcnt(wait_vmcnt(kFIns));  // B(kb)
+      }
+      __builtin_amdgcn_s_barrier();
+      if (!first) __builtin_amdgcn_s_barrier();  // one phase behind from here on
+      unsigned ast = 0, bst = 0;  // byte offsets of the k-tile's stages
       for (int kt = kb; kt < ke; ++kt) {
-        // A(kt) and B(kt) have landed; B(kt + 1), issued after A(kt), may be in flight.
+        // Read phase. A(kt + 1) goes to the stage A(kt - 1) used and B(kt + 2) to the one
+        // B(kt - 1) used: both groups have read those. Loads past the last k-tile land as
+        // zeros and keep the counts.
+        load(first ? kt + 1 : kt + 2,
+             first ? sA + (ast ^ kFTileBytes) : sB + (bst == 0 ? 2 * kFTileBytes : bst - kFTileBytes));
+        __builtin_amdgcn_sched_barrier(0);
+        bf16x8_t f[2 * (FA + FB)];
+        asm_frags<AMODE, BMODE, PAIRED, 0>(f, abase + ast, bbase + bst);
+        __builtin_amdgcn_sched_barrier(0);
+        // B(kt + 1) has landed (only the second group has older loads in flight here).
         __builtin_amdgcn_s_waitcnt(wait_vmcnt(kFIns));
+        tie_wait(f);
+        __builtin_amdgcn_sched_barrier(0);
+        // Before the first group's epilogue stages through LDS: no load may be in flight.
+        if (kt + 1 == ke) __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
         __builtin_amdgcn_s_barrier();
-        if (kt + 1 < ke)
-          la.issue(q.a, row0_a, (kt + 1) * kFBK, p.K, sA + ((kt - kb + 1) & 1) * kFTileBytes, wave, lane);
-        const unsigned char* sa = sA + ((kt - kb) & 1) * kFTileBytes;
-        const unsigned char* sb = sB + bst * kFTileBytes;
-        // B(kt + 2) goes to the stage B(kt - 1) used, which every wave has read (barrier).
-        unsigned char* const nb = sB + (bst == 0 ? 2 : bst - 1) * kFTileBytes;
-        bf16x8_t af[2][FA], bfr[2][FB];
-#pragma unroll
-        for (int i = 0; i < FA; ++i) af[0][i] = read_frag<AMODE>(sa, wm * TM + 16 * i, 0, lane);
-#pragma unroll
-        for (int j = 0; j < FB; ++j) bfr[0][j] = read_frag<BMODE>(sb, b_rb[j], 0, lane);
-#pragma unroll
-        for (int i = 0; i < FA; ++i) af[1][i] = read_frag<AMODE>(sa, wm * TM + 16 * i, 1, lane);
-#pragma unroll
-        for (int j = 0; j < FB; ++j) bfr[1][j] = read_frag<BMODE>(sb, b_rb[j], 1, lane);
-#pragma unroll
-        for (int i = 0; i < FA; ++i)
-#pragma unroll
-          for (int j = 0; j < FB; ++j)
-            acc.v[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[0][j], af[0][i], acc.v[i][j], 0, 0, 0);
-        // Step-0 reads first, then step 1's reads spread over step 0's MFMAs.
-        __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-          __builtin_amdgcn_sched_group_barrier(0x008, NM / NR > 0 ? NM / NR : 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, NM - (NM / NR > 0 ? NM / NR : 1) * NR, 0);
         __builtin_amdgcn_sched_barrier(0);
-        // B two tiles ahead, between the steps: it lands while step 1 reads nothing.
+        // MFMA phase.
 #pragma unroll
-        for (int i = 0; i < kFIns; ++i)
-          lb.issue_one(q.b, row0_b, (kt + 2) * kFBK, p.K, nb, wave, lane, i, kt + 2 < ke);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < FA; ++i)
-#pragma unroll
-          for (int j = 0; j < FB; ++j)
-            acc.v[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[1][j], af[1][i], acc.v[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
-        bst = bst == 2 ? 0 : bst + 1;
-      }
-      // The zero-filling loads of the last two k-tiles land, and every wave is done reading,
-      // before the epilogue's staging writes and the next tile's first loads.
-      __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
-      __builtin_amdgcn_s_barrier();
-    } else if (kb < ke && kBothMN) {
-      static_assert(FA + FB == 12, "tie_wait binds 12 fragments");
-      const unsigned lds0 =
-          (unsigned)(unsigned long)(__attribute__((address_space(3))) unsigned char*)fsmem;
-      unsigned abase[FA], bbase[FB];
-#pragma unroll
-      for (int i = 0; i < FA; ++i) abase[i] = lds0 + tr_base(wm * TM + 16 * i, lane);
-#pragma unroll
-      for (int j = 0; j < FB; ++j) bbase[j] = lds0 + kFTileBytes + tr_base(b_rb[j], lane);
-      la.issue(q.a, row0_a, kb * kFBK, p.K, fsmem, wave, lane);
-      lb.issue(q.b, row0_b, kb * kFBK, p.K, fsmem + kFTileBytes, wave, lane);
-      for (int kt = kb; kt < ke; ++kt) {
-        const int cur = (kt - kb) & 1;
-        __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
-        __builtin_amdgcn_s_barrier();
-        // The next tile's loads first: a full k-tile of lead.
-        if (kt + 1 < ke) {
-          unsigned char* nxt = fsmem + (cur ^ 1) * kFStageBytes;
-          la.issue(q.a, row0_a, (kt + 1) * kFBK, p.K, nxt, wave, lane);
-          lb.issue(q.b, row0_b, (kt + 1) * kFBK, p.K, nxt + kFTileBytes, wave, lane);
-        }
-        const unsigned st = (unsigned)(cur * kFStageBytes);
-        __builtin_amdgcn_sched_barrier(0);
-        bf16x8_t f0[FA + FB], f1[FA + FB];  // steps 0 and 1: A blocks, then B blocks
-#pragma unroll
-        for (int i = 0; i < FA; ++i) f0[i] = tr_frag<0>(abase[i] + st);
-#pragma unroll
-        for (int j = 0; j < FB; ++j) f0[FA + j] = tr_frag<0>(bbase[j] + st);
-        tie_wait(f0);
-        __builtin_amdgcn_sched_barrier(0);
-        // Step 0's MFMAs, step 1's fragment r read after MFMA ceil(r NM / 12).
-#pragma unroll
-        for (int n = 0; n < NM; ++n) {
-          const int i = n / FB, j = n % FB;
-          acc.v[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f0[FA + j], f0[i], acc.v[i][j], 0, 0, 0);
-          if ((n * (FA + FB)) % NM < FA + FB) {
-            const int r = n * (FA + FB) / NM;
-            f1[r] = r < FA ? tr_frag<1>(abase[r] + st) : tr_frag<1>(bbase[r - FA] + st);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        tie_wait(f1);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < FA; ++i)
-#pragma unroll
-          for (int j = 0; j < FB; ++j)
-            acc.v[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f1[FA + j], f1[i], acc.v[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      // All waves are done reading both stages before the next tile's first load.
-      __builtin_amdgcn_s_barrier();
-    } else if (kb < ke) {
-      la.issue(q.a, row0_a, kb * kFBK, p.K, fsmem, wave, lane);
-      lb.issue(q.b, row0_b, kb * kFBK, p.K, fsmem + kFTileBytes, wave, lane);
-      for (int kt = kb; kt < ke; ++kt) {
-        const int cur = (kt - kb) & 1;
-        __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
-        __builtin_amdgcn_s_barrier();
-        const unsigned char* sa = fsmem + cur * kFStageBytes;
-        const unsigned char* sb = sa + kFTileBytes;
-        bf16x8_t af[2][FA], bfr[2][FB];
-#pragma unroll
-        for (int i = 0; i < FA; ++i) af[0][i] = read_frag<AMODE>(sa, wm * TM + 16 * i, 0, lane);
-#pragma unroll
-        for (int j = 0; j < FB; ++j) bfr[0][j] = read_frag<BMODE>(sb, b_rb[j], 0, lane);
-#pragma unroll
-        for (int s = 0; s < kFBK / 32; ++s) {
-          if (s == 1) {
-            // Step-0 reads first, then step 1's reads spread over step 0's MFMAs; then the
-            // next k-tile's loads, after this wave's last fragment read of the tile.
-            __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
-#pragma unroll
-            for (int r = 0; r < NR; ++r) {
-              __builtin_amdgcn_sched_group_barrier(0x008, NM / NR > 0 ? NM / NR : 1, 0);
-              __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x008, NM - (NM / NR > 0 ? NM / NR : 1) * NR, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            if (kt + 1 < ke) {
-              unsigned char* nxt = fsmem + (cur ^ 1) * kFStageBytes;
-              la.issue(q.a, row0_a, (kt + 1) * kFBK, p.K, nxt, wave, lane);
-              lb.issue(q.b, row0_b, (kt + 1) * kFBK, p.K, nxt + kFTileBytes, wave, lane);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          if (s + 1 < kFBK / 32) {
-#pragma unroll
-            for (int i = 0; i < FA; ++i) af[(s + 1) & 1][i] = read_frag<AMODE>(sa, wm * TM + 16 * i, s + 1, lane);
-#pragma unroll
-            for (int j = 0; j < FB; ++j) bfr[(s + 1) & 1][j] = read_frag<BMODE>(sb, b_rb[j], s + 1, lane);
-          }
+        for (int s = 0; s < 2; ++s)
 #pragma unroll
           for (int i = 0; i < FA; ++i)
 #pragma unroll
             for (int j = 0; j < FB; ++j)
-              acc.v[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[s & 1][j], af[s & 1][i],
+              acc.v[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[12 * s + FA + j], f[12 * s + i],
                                                                      acc.v[i][j], 0, 0, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (first) __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));  // A(kt + 1) has landed
+        // The second group's last MFMA phase ends the loop: the first group is past it.
+        if (first || kt + 1 < ke) __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        ast ^= kFTileBytes;
+        bst = bst == 2 * kFTileBytes ? 0 : bst + kFTileBytes;
       }
-      // All waves are done reading both stages before the next tile's first load.
-      __builtin_amdgcn_s_barrier();
     }
     const int m_base = row0_a + wm * TM;
     const int n_base = row0_b + (PAIRED ? wn * (TN / 2) : wn * TN);

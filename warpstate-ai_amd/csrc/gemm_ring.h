@@ -16,71 +16,6 @@
 
 namespace ws {
 
-// 16 bytes per lane from `rs` at byte offset `off` into LDS at lds + 16 * lane. (A function
-// of its own: with template-dependent arguments the builtin's target check fails on the
-// compiler's host pass.)
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, unsigned char* lds, unsigned off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, WS_LDS(lds), 16, off, 0, 0, 0);
-}
-
-// Direct-to-LDS loader of a ROWS x 64 operand tile by NT threads, in the tile layouts of
-// gemm_fast.h (K-contiguous: [ROWS][64 k] with swizzled 16-byte chunks; M/N-contiguous:
-// blocks of 64 operand rows, each [64 k][128 B]).
-template <int ROWS, int NT, int MODE, bool PAIRED>
-struct RingTile {
-  static constexpr int kIns = ROWS * 8 / NT;
-  static_assert(kIns >= 1 && ROWS * 8 % NT == 0 && ROWS % 64 == 0, "whole loads per thread");
-  unsigned off[kIns];
-
-  __device__ __forceinline__ static int k_of(int i, int wave, int lane) {
-    const int byte = (i * (NT / kWave) + wave) * 1024 + lane * 16;
-    if constexpr (MODE == kKContig) return 8 * (((byte >> 4) & 7) ^ swz(byte >> 7));
-    else return ((byte >> 10) & 7) * 8 + (lane >> 3);
-  }
-  __device__ __forceinline__ void init(const OperandDesc& d, int row0, int rows_valid, int half,
-                                       int wave, int lane) {
-#pragma unroll
-    for (int i = 0; i < kIns; ++i) {
-      const int byte = (i * (NT / kWave) + wave) * 1024 + lane * 16;
-      int r, c = 0, kk = 0;
-      if constexpr (MODE == kKContig) {
-        r = byte >> 7;
-        c = ((byte >> 4) & 7) ^ swz(r);
-      } else {
-        const int q = byte >> 10;
-        kk = (q & 7) * 8 + (lane >> 3);
-        r = (q >> 3) * 64 + 8 * ((lane & 7) ^ mnsw(kk));  // first operand row of the chunk
-      }
-      const int logical = row0 + (PAIRED && r >= ROWS / 2 ? r - ROWS / 2 : r);
-      const int phys = PAIRED && r >= ROWS / 2 ? half + logical : logical;
-      const long rel = MODE == kKContig ? (long)(phys - row0) * d.s_row * 2 + 16 * c
-                                        : (phys - row0) * 2 + (long)kk * d.s_k * 2;
-      off[i] = logical < rows_valid ? (unsigned)rel : kOOB;
-    }
-  }
-  // The tile at k0 into `lds_tile`; chunks at k >= K (all of them past the last k-tile)
-  // land as zeros, so that every wait counts the same number of loads.
-  __device__ __forceinline__ void issue(const OperandDesc& d, int row0, int k0, int K,
-                                        unsigned char* lds_tile, int wave, int lane) const {
-    const unsigned short* base =
-        MODE == kKContig ? d.ptr + (long)row0 * d.s_row + k0 : d.ptr + row0 + (long)k0 * d.s_k;
-    __amdgpu_buffer_rsrc_t rs = make_rsrc(base, 0x7fffffff);
-    if (k0 + kFBK <= K) {
-#pragma unroll
-      for (int i = 0; i < kIns; ++i)
-        dma16(rs, lds_tile + (i * (NT / kWave) + wave) * 1024, off[i]);
-    } else {
-      int l = lane;
-      asm volatile("" : "+v"(l));
-#pragma unroll
-      for (int i = 0; i < kIns; ++i) {
-        const unsigned o = k0 + k_of(i, wave, l) >= K ? kOOB : off[i];
-        dma16(rs, lds_tile + (i * (NT / kWave) + wave) * 1024, o);
-      }
-    }
-  }
-};
-
 // A wait for every LDS read issued so far that also redefines the N fragment registers, so
 // that no MFMA reading them can be scheduled ahead of it (tie_wait of gemm_fast.h).
 template <int N>
@@ -95,15 +30,6 @@ __device__ __forceinline__ void tie_frags(bf16x8_t (&f)[N]) {
     asm volatile("s_waitcnt lgkmcnt(0)"
                  : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]), "+v"(f[6]),
                    "+v"(f[7])::"memory");
-}
-
-// One K-contiguous fragment read as inline assembly (read_frag<kKContig>), for loops whose
-// other operand uses the transposing assembly reads.
-template <int OFF>
-__device__ __forceinline__ bf16x8_t b128_read(unsigned addr) {
-  u32x4_t v;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "i"(OFF) : "memory");
-  return __builtin_bit_cast(bf16x8_t, v);
 }
 
 // Macro-tile of the ring kernel: BM x BN outputs on WM x WN waves, S LDS stages.
@@ -251,9 +177,9 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_ring_kernel(const GemmParams p) 
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
 #pragma unroll
-          for (int i = 0; i < FA; ++i) af[s][i] = read_frag<AMODE>(sa, wm * TM + 16 * i, s, lane);
+          for (int i = 0; i < FA; ++i) af[s][i] = read_frag(sa, wm * TM + 16 * i, s, lane);
 #pragma unroll
-          for (int j = 0; j < FB; ++j) bf[s][j] = read_frag<BMODE>(sb, b_rb[j], s, lane);
+          for (int j = 0; j < FB; ++j) bf[s][j] = read_frag(sb, b_rb[j], s, lane);
         }
 #pragma unroll
         for (int s = 0; s < 2; ++s)

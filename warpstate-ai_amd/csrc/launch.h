@@ -135,8 +135,7 @@ inline int check_out_stride(long ld, int elem_bytes, const char* what) {
 template <int AM, int BMD, bool PAIRED, class Epi>
 int run_fast(GemmParams p, LaunchCfg cfg, hipStream_t stream) {
   const void* kern = reinterpret_cast<const void*>(&gemm_fast_kernel<AM, BMD, PAIRED, Epi>);
-  constexpr int lds_bytes = fast_lds_bytes<AM, BMD>();
-  if (int rc = ensure_lds(kern, lds_bytes)) return rc;
+  if (int rc = ensure_lds(kern, kFLdsBytes)) return rc;
   const int cols = PAIRED ? p.H : p.N;
   const int bn_cols = PAIRED ? kFBN / 2 : kFBN;
   p.tiles_m = cdiv(p.M, kFBM);
@@ -150,7 +149,7 @@ int run_fast(GemmParams p, LaunchCfg cfg, hipStream_t stream) {
   dim3 grid(cfg.persistent ? (p.total_tiles < resident ? p.total_tiles : resident) : p.total_tiles,
             splits);
   if (cfg.workers > 0) grid = dim3(cfg.workers, 1);
-  hipLaunchKernelGGL((gemm_fast_kernel<AM, BMD, PAIRED, Epi>), grid, dim3(kFNT), lds_bytes, stream, p);
+  hipLaunchKernelGGL((gemm_fast_kernel<AM, BMD, PAIRED, Epi>), grid, dim3(kFNT), kFLdsBytes, stream, p);
   return hip_check(hipGetLastError(), "gemm launch");
 }
 
@@ -194,10 +193,11 @@ enum FastTile { kTile256 = 0, kTile128x2, kTile128x1, kTile64x128, kTile64, kFas
 // 64-deep k-tile for one workgroup, `pair` us for two that share the CU, and `fixed` us
 // around the k-loop. The 256 x 256 tile costs less per product with every CU busy; below about
 // one round of its tiles most CUs idle, and a smaller tile wins although it loads its operands
-// more often. Measured, us (256 x 256 against the choice): 512 x 1280 x 8960 159 / 40
-// (64 x 64), 1999 x 1280 x 8960 158 / 71 (128 x 128 alone), 4096 x 1280 x 6400 114 / 71
-// (128 x 128 paired), 128 x 4800 x 960 23 / 7.4 (64 x 64); and where it stays: 8192 x 10240 x
-// 2048 250 / 294, 8192 x 2048 x 2048 54 / 59 (the best smaller tile).
+// more often. Measured, us (256 x 256 against the choice): 1999 x 1280 x 8960 136 / 71 (128 x
+// 128 alone), 4096 x 2048 x 5632 95 / 78 (128 x 128 paired), 1999 x 8960 x 1280 59 / 53; with
+// the 256 x 256 tile's former loop, 4-14 % slower: 512 x 1280 x 8960 159 / 40 (64 x 64), 128 x
+// 4800 x 960 23 / 7.4 (64 x 64); and where it stays: 8192 x 10240 x 2048 245 / 298, 8192 x
+// 2048 x 2048 51 / 59 (the best smaller tile).
 struct TileCost {
   int bm, bn;
   float alone, pair, fixed;  // pair 0: one workgroup per CU
@@ -210,19 +210,19 @@ struct TileCost {
 };
 inline const TileCost& tile_cost(int tile, int am, int bm) {
   static const TileCost kk[kFastTiles] = {
-      {256, 256, 1.55f, 0.0f, 4.0f, 0, 0, 0, 1.05f, 5.0f},
+      {256, 256, 1.43f, 0.0f, 4.0f, 0, 0, 0, 1.05f, 5.0f},
       {128, 128, 0.62f, 0.87f, 3.2f, 0.07f, 0.006f, 0.18f, 1.25f, 5.0f},
       {128, 128, 0.50f, 0.0f, 3.6f, 0, 0, 0, 1.1f, 1.7f},
       {64, 128, 0.34f, 0.50f, 3.6f, 0.0f, 0.005f, 0.16f, 1.2f, 1.0f},
       {64, 64, 0.28f, 0.33f, 3.4f, 0.0f, 0.0015f, 0.09f, 1.4f, 0.5f}};
   static const TileCost kmn[kFastTiles] = {
-      {256, 256, 1.87f, 0.0f, 4.0f, 0, 0, 0, 1.05f, 5.0f},
+      {256, 256, 1.48f, 0.0f, 4.0f, 0, 0, 0, 1.05f, 5.0f},
       {128, 128, 0.64f, 0.89f, 3.2f, 0.07f, 0.006f, 0.18f, 1.25f, 5.0f},
       {128, 128, 0.53f, 0.0f, 3.6f, 0, 0, 0, 1.1f, 1.7f},
       {64, 128, 0.38f, 0.53f, 3.6f, 0.0f, 0.005f, 0.16f, 1.2f, 1.0f},
       {64, 64, 0.31f, 0.36f, 3.4f, 0.0f, 0.0015f, 0.09f, 1.4f, 0.5f}};
   static const TileCost mnmn[kFastTiles] = {
-      {256, 256, 1.85f, 0.0f, 4.0f, 0, 0, 0, 1.0f, 5.0f},
+      {256, 256, 1.52f, 0.0f, 4.0f, 0, 0, 0, 1.0f, 5.0f},
       {128, 128, 0.60f, 1.00f, 3.2f, 0, 0, 0, 1.0f, 5.0f},
       {128, 128, 0.54f, 0.0f, 3.6f, 0, 0, 0, 1.0f, 1.7f},
       {64, 128, 0.39f, 0.70f, 3.6f, 0, 0, 0, 1.0f, 1.0f},
@@ -251,7 +251,7 @@ inline float tile_time(int tile, long m, long n, long k, int am, int bm, int cus
     if (tile != kTile256) return (float)(rounds + (rest != 0)) * (alone * kt + fixed + epi * area);
     // With most CUs idle in the last round its tiles' loads meet less traffic.
     float t = (float)rounds * (alone * kt + fixed + epi);
-    if (rest) t += alone * (0.73f + 0.27f * (float)rest / (float)cus) * kt + fixed + epi;
+    if (rest) t += alone * (0.65f + 0.30f * (float)rest / (float)cus) * kt + fixed + epi;
     return t;
   }
   const long rounds = tiles / (2 * cus), rest = tiles % (2 * cus);

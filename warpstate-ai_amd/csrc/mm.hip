@@ -58,19 +58,6 @@ extern "C" int ws_mm(const void* a, int64_t a_s0, int64_t a_s1, const void* b, i
   return dispatch<kMaskMM, WS_TILE_ARGS_SMALL, false, EpiStore<false, false>>(p, am, bm, cfg, s);
 }
 
-// Copying B [k, n] K-contiguous costs about 3 us and 4 n k bytes at 5.5 TB/s; the 256 x 256
-// tile gains 20 % from it, the smaller ones 2-5 %. Measured with and without the copy, us:
-// 16384 x 2048 x 11264 546 / 646, 8192 x 1280 x 6400 133 / 178, 4096 x 1280 x 6400 83 / 74,
-// 1999 x 1280 x 8960 82 / 75, 512 x 1280 x 8960 51 / 44.
-extern "C" int ws_mm_copy_pays(int64_t m, int64_t n, int64_t k, int swiglu_backward) {
-  if (m < 1 || n < 1 || k < 1 || !fits_i32(m) || !fits_i32(n) || !fits_i32(k)) return 0;
-  const float epi = swiglu_backward ? kEpiSwigluBwd : kEpiStore;
-  float direct, copied;
-  pick_tile(m, n, k, kKContig, kMNContig, false, epi, &direct);
-  pick_tile(m, n, k, kKContig, kKContig, false, epi, &copied);
-  return copied + 3.0f + 4.0f * (float)n * (float)k / 5.5e6f < direct;
-}
-
 extern "C" int ws_swiglu_mm(const void* a, int64_t a_s0, int64_t a_s1, const void* b,
                             int64_t b_s0, int64_t b_s1, void* packed, void* act, int64_t m,
                             int64_t h, int64_t k, int eager_rounding, int algorithm, int tile,

@@ -28,7 +28,6 @@ SIGNATURES = {
     "ws_version": (ctypes.c_char_p, []),
     "ws_mm": (_i32, [_c_void_p, _i64, _i64, _c_void_p, _i64, _i64, _c_void_p, _i64, _i64, _i64,
                      _i32, _i32, _c_void_p]),
-    "ws_mm_copy_pays": (_i32, [_i64, _i64, _i64, _i32]),
     "ws_swiglu_mm": (_i32, [_c_void_p, _i64, _i64, _c_void_p, _i64, _i64, _c_void_p, _c_void_p,
                             _i64, _i64, _i64, _i32, _i32, _i32, _c_void_p]),
     "ws_swiglu_forward": (_i32, [_c_void_p, _c_void_p, _i64, _i64, _i32, _c_void_p]),

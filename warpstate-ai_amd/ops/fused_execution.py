@@ -86,21 +86,25 @@ def k_contiguous_b(b: torch.Tensor, rows_a: int) -> torch.Tensor:
     return b
 
 
-def gemm_b(a: torch.Tensor, b: torch.Tensor, swiglu_backward: bool = False) -> torch.Tensor:
-    """B [K, N] as the GEMM of ``a`` [M, K] best reads it: ``k_contiguous_b``'s copy, or B
-    itself where the vector loaders read an N-contiguous B directly at no loss: beside a
-    token-major A (a weight gradient's dY.T: both operands go through the same transposing
-    loop; 10240 x 2048 x 8192 takes 421 us with a copied B, 300 without) and for products
-    that the library expects to gain less than the copy costs (``ws_mm_copy_pays``). Same
-    bits."""
-    k, n = b.shape
+# Rows of A from which the GEMM reads a K-contiguous copy of B although the vector loaders take
+# an N-contiguous B. The product gains 2-4 % and the copy costs as much: 16384 x 2048 x 11264
+# 508 + 14 us against 519; below, the copy only loses (8192 x 1280 x 6400 111 + 8 against 113,
+# 4096 x 1280 x 6400 75 + 7 against 74).
+DIRECT_MAX_ROWS = 16384
+
+
+def gemm_b(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+    """B [K, N] as the GEMM of ``a`` [M, K] reads it: ``k_contiguous_b``'s copy, or B itself
+    where the vector loaders read an N-contiguous B directly at no loss: below
+    ``DIRECT_MAX_ROWS`` rows, and beside a token-major A (a weight gradient's dY.T: both
+    operands go through the transposing reads). Same bits."""
+    m, n = a.shape[0], b.shape[1]
     if b.stride(1) == 1 and n % 8 == 0 and b.stride(0) % 8 == 0 and b.data_ptr() % 16 == 0:
-        token_major = (a.stride(0) == 1 and a.shape[0] % 8 == 0 and a.stride(1) % 8 == 0
+        token_major = (a.stride(0) == 1 and m % 8 == 0 and a.stride(1) % 8 == 0
                        and a.data_ptr() % 16 == 0)
-        if token_major or not _hip.query("ws_mm_copy_pays", a.shape[0], n, k,
-                                         int(swiglu_backward)):
+        if token_major or m < DIRECT_MAX_ROWS:
             return b
-    return k_contiguous_b(b, a.shape[0])
+    return k_contiguous_b(b, m)
 
 
 def mm(a: torch.Tensor, b: torch.Tensor, algorithm: str = "tiled", tile: int = 0) -> torch.Tensor:
@@ -249,10 +253,7 @@ def swiglu_backward_mm(grad: torch.Tensor, down_weight: torch.Tensor, packed: to
     if out is None:
         out = torch.empty((m, 2 * h), dtype=torch.bfloat16, device=grad.device)
     _check_buffer(out, (m, 2 * h), torch.bfloat16, grad.device, "out")
-    # From 16384 rows the 256 x 256 tiles on a copy and the paired 128 x 128 ones on the weight
-    # itself are level (h 5632, d 2048: 401-425 + 14 us against 421); below, the copy loses.
-    down_weight = (k_contiguous_b(down_weight, m) if m >= 16384
-                   else gemm_b(grad, down_weight, True))
+    down_weight = gemm_b(grad, down_weight)
     _hip.call("ws_swiglu_backward_mm", grad.data_ptr(), grad.stride(0), grad.stride(1),
               down_weight.data_ptr(), down_weight.stride(0), down_weight.stride(1),
               packed.data_ptr(), out.data_ptr(), m, h, k, int(eager_rounding), _hip.stream(grad))
