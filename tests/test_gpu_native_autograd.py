@@ -83,3 +83,19 @@ def test_saved_tensor_hooks_see_every_saved_tensor(name):
                     torch.autograd.grad(plain, leaves, grad)):
         assert torch.equal(g, e), name
     assert packed
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_calls_that_record_nothing_take_forward_mode_tensors(name):
+    import torch.autograd.forward_ad as fwad
+
+    op, leaves, rest = _case(name)
+    want = op(*leaves, *rest)
+    want = want[0] if isinstance(want, tuple) else want
+    plain = [t.detach() for t in leaves]
+    with fwad.dual_level():
+        got = op(fwad.make_dual(plain[0], torch.ones_like(plain[0])), *plain[1:], *rest)
+        got = got[0] if isinstance(got, tuple) else got
+        primal, tangent = fwad.unpack_dual(got)
+        assert tangent is None and not primal.requires_grad
+        assert torch.equal(primal, want.detach())

@@ -10,8 +10,10 @@
 // (86 us per pass of the 16384 x 2048 x 5632 SwiGLU block).
 //
 // They dispatch below autograd and nothing else: fake tensors, tracing, functorch and
-// saved-tensor hooks see the operators as before. A backward under create_graph goes through
-// the backward operator's own autograd kernel, which refuses to be differentiated.
+// saved-tensor hooks see the operators as before. A call that records nothing (no_grad, or no
+// input that requires a gradient) goes straight to the operator's kernel, as the Python
+// functions do: a node would refuse forward-mode tensors there. A backward under create_graph
+// goes through the backward operator's own autograd kernel, which refuses to be differentiated.
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
 
@@ -33,6 +35,11 @@ auto below(const Op& op, Args&&... args) {
   at::AutoDispatchBelowAutograd guard;
   return op.call(std::forward<Args>(args)...);
 }
+// Whether a call with these inputs records a node.
+template <class... Inputs>
+bool records(const Inputs&... inputs) {
+  return at::GradMode::is_enabled() && (inputs.requires_grad() || ...);
+}
 // A backward operator: below autograd, unless its own gradient is being recorded.
 template <class Op, class... Args>
 auto backward_op(const Op& op, Args&&... args) {
@@ -46,9 +53,12 @@ Tensor grad_or_zeros(const Tensor& grad, const Tensor& like, c10::SymIntArrayRef
 }
 
 struct SwigluFn : Function<SwigluFn> {
+  static const auto& op() {
+    static const auto handle = find<Tensor(const Tensor&, bool)>("warpstate::bf16_swiglu");
+    return handle;
+  }
   static Tensor forward(AutogradContext* ctx, const Tensor& packed, bool eager) {
-    static auto op = find<Tensor(const Tensor&, bool)>("warpstate::bf16_swiglu");
-    Tensor out = below(op, packed, eager);
+    Tensor out = below(op(), packed, eager);
     ctx->save_for_backward({packed});
     ctx->saved_data["eager"] = eager;
     return out;
@@ -61,12 +71,16 @@ struct SwigluFn : Function<SwigluFn> {
 };
 
 struct RmsnormFn : Function<RmsnormFn> {
+  static const auto& op() {
+    static const auto handle =
+        find<std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, double, bool)>(
+            "warpstate::bf16_rmsnorm");
+    return handle;
+  }
   static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight,
                                double eps, bool eager) {
-    static auto op = find<std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, double, bool)>(
-        "warpstate::bf16_rmsnorm");
     ctx->set_materialize_grads(false);
-    auto [y, rstd] = below(op, x, weight, eps, eager);
+    auto [y, rstd] = below(op(), x, weight, eps, eager);
     ctx->save_for_backward({x, weight, rstd});
     ctx->mark_non_differentiable({rstd});
     ctx->saved_data["eager"] = eager;
@@ -86,13 +100,17 @@ struct RmsnormFn : Function<RmsnormFn> {
 
 struct NormProjectionFn : Function<NormProjectionFn> {
   typedef std::tuple<Tensor, Tensor, Tensor, Tensor> Out;
+  static const auto& op() {
+    static const auto handle = find<Out(const Tensor&, const Tensor&, const Tensor&, double,
+                                        c10::SymInt, c10::SymInt)>(
+        "warpstate::fused_norm_projection");
+    return handle;
+  }
   static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& norm_weight,
                                const Tensor& weight, double eps, c10::SymInt gate_begin,
                                c10::SymInt gate_end) {
-    static auto op = find<Out(const Tensor&, const Tensor&, const Tensor&, double, c10::SymInt,
-                              c10::SymInt)>("warpstate::fused_norm_projection");
     ctx->set_materialize_grads(false);
-    auto [out, rstd, normed, w] = below(op, x, norm_weight, weight, eps, gate_begin, gate_end);
+    auto [out, rstd, normed, w] = below(op(), x, norm_weight, weight, eps, gate_begin, gate_end);
     ctx->save_for_backward({x, norm_weight, rstd, normed, w, out});
     ctx->saved_data["gate_begin"] = gate_begin;
     ctx->saved_data["gate_end"] = gate_end;
@@ -122,12 +140,16 @@ variable_list projection_grads(const char* name, const Tensor& grad, const Tenso
 }
 
 struct ResidualProjectionFn : Function<ResidualProjectionFn> {
+  static const auto& op() {
+    static const auto handle =
+        find<std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&)>(
+            "warpstate::fused_residual_projection");
+    return handle;
+  }
   static variable_list forward(AutogradContext* ctx, const Tensor& a, const Tensor& weight,
                                const Tensor& residual) {
-    static auto op = find<std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&)>(
-        "warpstate::fused_residual_projection");
     ctx->set_materialize_grads(false);
-    auto [out, w] = below(op, a, weight, residual);
+    auto [out, w] = below(op(), a, weight, residual);
     ctx->save_for_backward({a, w});
     return {out, w};
   }
@@ -141,11 +163,14 @@ struct ResidualProjectionFn : Function<ResidualProjectionFn> {
 };
 
 struct LinearFn : Function<LinearFn> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& a, const Tensor& weight) {
-    static auto op = find<std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&)>(
+  static const auto& op() {
+    static const auto handle = find<std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&)>(
         "warpstate::fused_linear");
+    return handle;
+  }
+  static variable_list forward(AutogradContext* ctx, const Tensor& a, const Tensor& weight) {
     ctx->set_materialize_grads(false);
-    auto [out, w] = below(op, a, weight);
+    auto [out, w] = below(op(), a, weight);
     ctx->save_for_backward({a, w});
     return {out, w};
   }
@@ -173,12 +198,16 @@ Tensor swiglu_block_grad(const variable_list& grads, const variable_list& s) {
 }
 
 struct SwigluBlockFn : Function<SwigluBlockFn> {
+  static const auto& op() {
+    static const auto handle =
+        find<FiveTensors(const Tensor&, const Tensor&, const Tensor&, const Tensor&)>(
+            "warpstate::fused_swiglu_block");
+    return handle;
+  }
   static variable_list forward(AutogradContext* ctx, const Tensor& h, const Tensor& w_upgate,
                                const Tensor& w_down, const Tensor& residual) {
-    static auto op = find<FiveTensors(const Tensor&, const Tensor&, const Tensor&, const Tensor&)>(
-        "warpstate::fused_swiglu_block");
     ctx->set_materialize_grads(false);
-    auto [out, packed, act, wug, wd] = below(op, h, w_upgate, w_down, residual);
+    auto [out, packed, act, wug, wd] = below(op(), h, w_upgate, w_down, residual);
     ctx->save_for_backward({h, packed, act, wug, wd});
     return {out, packed, act, wug, wd};
   }
@@ -191,12 +220,15 @@ struct SwigluBlockFn : Function<SwigluBlockFn> {
 };
 
 struct SwigluMlpFn : Function<SwigluMlpFn> {
+  static const auto& op() {
+    static const auto handle = find<FiveTensors(const Tensor&, const Tensor&, const Tensor&)>(
+        "warpstate::fused_swiglu_mlp");
+    return handle;
+  }
   static variable_list forward(AutogradContext* ctx, const Tensor& h, const Tensor& w_upgate,
                                const Tensor& w_down) {
-    static auto op = find<FiveTensors(const Tensor&, const Tensor&, const Tensor&)>(
-        "warpstate::fused_swiglu_mlp");
     ctx->set_materialize_grads(false);
-    auto [out, packed, act, wug, wd] = below(op, h, w_upgate, w_down);
+    auto [out, packed, act, wug, wd] = below(op(), h, w_upgate, w_down);
     ctx->save_for_backward({h, packed, act, wug, wd});
     return {out, packed, act, wug, wd};
   }
@@ -212,8 +244,12 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> four(const variable_list& v) {
 }
 FiveTensors five(const variable_list& v) { return {v[0], v[1], v[2], v[3], v[4]}; }
 
-Tensor swiglu(const Tensor& packed, bool eager) { return SwigluFn::apply(packed, eager); }
+Tensor swiglu(const Tensor& packed, bool eager) {
+  if (!records(packed)) return below(SwigluFn::op(), packed, eager);
+  return SwigluFn::apply(packed, eager);
+}
 std::tuple<Tensor, Tensor> rmsnorm(const Tensor& x, const Tensor& weight, double eps, bool eager) {
+  if (!records(x, weight)) return below(RmsnormFn::op(), x, weight, eps, eager);
   return two(RmsnormFn::apply(x, weight, eps, eager));
 }
 std::tuple<Tensor, Tensor, Tensor, Tensor> norm_projection(const Tensor& x,
@@ -221,20 +257,27 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> norm_projection(const Tensor& x,
                                                            const Tensor& weight, double eps,
                                                            c10::SymInt gate_begin,
                                                            c10::SymInt gate_end) {
+  if (!records(x, norm_weight, weight))
+    return below(NormProjectionFn::op(), x, norm_weight, weight, eps, gate_begin, gate_end);
   return four(NormProjectionFn::apply(x, norm_weight, weight, eps, gate_begin, gate_end));
 }
 std::tuple<Tensor, Tensor> residual_projection(const Tensor& a, const Tensor& weight,
                                                const Tensor& residual) {
+  if (!records(a, weight, residual)) return below(ResidualProjectionFn::op(), a, weight, residual);
   return two(ResidualProjectionFn::apply(a, weight, residual));
 }
 std::tuple<Tensor, Tensor> linear(const Tensor& a, const Tensor& weight) {
+  if (!records(a, weight)) return below(LinearFn::op(), a, weight);
   return two(LinearFn::apply(a, weight));
 }
 FiveTensors swiglu_block(const Tensor& h, const Tensor& w_upgate, const Tensor& w_down,
                          const Tensor& residual) {
+  if (!records(h, w_upgate, w_down, residual))
+    return below(SwigluBlockFn::op(), h, w_upgate, w_down, residual);
   return five(SwigluBlockFn::apply(h, w_upgate, w_down, residual));
 }
 FiveTensors swiglu_mlp(const Tensor& h, const Tensor& w_upgate, const Tensor& w_down) {
+  if (!records(h, w_upgate, w_down)) return below(SwigluMlpFn::op(), h, w_upgate, w_down);
   return five(SwigluMlpFn::apply(h, w_upgate, w_down));
 }
 
