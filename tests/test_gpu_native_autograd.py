@@ -99,3 +99,33 @@ def test_calls_that_record_nothing_take_forward_mode_tensors(name):
         primal, tangent = fwad.unpack_dual(got)
         assert tangent is None and not primal.requires_grad
         assert torch.equal(primal, want.detach())
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_compiled_autograd_traces_the_native_nodes(name):
+    """A backward under compiled autograd, of an eager and of a compiled call, gives the
+    eager gradients."""
+    from torch._dynamo import compiled_autograd
+
+    op, leaves, rest = _case(name)
+
+    def call(*inputs):
+        out = op(*inputs, *rest)
+        return out[0] if isinstance(out, tuple) else out
+
+    def gradients(fn, grad):
+        for t in leaves:
+            t.grad = None
+        fn(*leaves).backward(grad)
+        return [t.grad for t in leaves]
+
+    torch._dynamo.reset()
+    try:
+        grad = torch.randn_like(call(*leaves))
+        want = gradients(call, grad)
+        for fn in (call, torch.compile(call, backend="aot_eager", fullgraph=True)):
+            with compiled_autograd._enable(torch.compile(backend="aot_eager")):
+                got = gradients(fn, grad)
+            assert all(torch.equal(a, b) for a, b in zip(want, got)), name
+    finally:
+        torch._dynamo.reset()

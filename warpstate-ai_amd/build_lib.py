@@ -43,14 +43,19 @@ def _compile(source: Path) -> Path:
     return obj
 
 
-def _build_autograd() -> Path:
-    """The C++ autograd kernels: host code against PyTorch's headers, no device code."""
+def autograd_command(source: Path, target: Path) -> list[str]:
+    """The host compiler's command for the C++ autograd kernels: PyTorch's headers, no device
+    code."""
     torch_dir = Path(importlib.util.find_spec("torch").origin).parent
     include = torch_dir / "include"
+    return [CXX, "-O2", "-std=c++17", "-fPIC", "-shared", f"-I{include}",
+            f"-I{include / 'torch' / 'csrc' / 'api' / 'include'}", str(source), "-o", str(target),
+            f"-L{torch_dir / 'lib'}", "-ltorch", "-ltorch_cpu", "-lc10"]
+
+
+def _build_autograd() -> Path:
     staging = AUTOGRAD.with_name(AUTOGRAD.name + ".tmp")
-    cmd = [CXX, "-O2", "-std=c++17", "-fPIC", "-shared", f"-I{include}",
-           f"-I{include / 'torch' / 'csrc' / 'api' / 'include'}", str(CSRC / "autograd.cpp"),
-           "-o", str(staging), f"-L{torch_dir / 'lib'}", "-ltorch", "-ltorch_cpu", "-lc10"]
+    cmd = autograd_command(CSRC / "autograd.cpp", staging)
     result = subprocess.run(cmd, capture_output=True, text=True)
     if result.returncode != 0:
         raise RuntimeError(f"{CXX} failed for autograd.cpp:\n{result.stderr}")

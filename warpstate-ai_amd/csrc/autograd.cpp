@@ -77,14 +77,16 @@ struct RmsnormFn : Function<RmsnormFn> {
             "warpstate::bf16_rmsnorm");
     return handle;
   }
-  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight,
-                               double eps, bool eager) {
+  // The statistics go out beside the node's one output, a tensor without history: an output
+  // marked non-differentiable would be refused by compiled autograd.
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, double eps,
+                        bool eager, Tensor* rstd_out) {
     ctx->set_materialize_grads(false);
     auto [y, rstd] = below(op(), x, weight, eps, eager);
     ctx->save_for_backward({x, weight, rstd});
-    ctx->mark_non_differentiable({rstd});
     ctx->saved_data["eager"] = eager;
-    return {y, rstd};
+    *rstd_out = rstd;
+    return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     static auto op = find<std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&,
@@ -94,7 +96,7 @@ struct RmsnormFn : Function<RmsnormFn> {
     auto [dx, dw] = backward_op(op, s[0], s[1], s[2],
                                 grad_or_zeros(grads[0], s[0], s[0].sym_sizes()),
                                 ctx->saved_data["eager"].toBool());
-    return {dx, dw, Tensor(), Tensor()};
+    return {dx, dw, Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -250,7 +252,9 @@ Tensor swiglu(const Tensor& packed, bool eager) {
 }
 std::tuple<Tensor, Tensor> rmsnorm(const Tensor& x, const Tensor& weight, double eps, bool eager) {
   if (!records(x, weight)) return below(RmsnormFn::op(), x, weight, eps, eager);
-  return two(RmsnormFn::apply(x, weight, eps, eager));
+  Tensor rstd;
+  Tensor y = RmsnormFn::apply(x, weight, eps, eager, &rstd);
+  return {y, rstd};
 }
 std::tuple<Tensor, Tensor, Tensor, Tensor> norm_projection(const Tensor& x,
                                                            const Tensor& norm_weight,
