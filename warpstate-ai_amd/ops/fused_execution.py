@@ -87,24 +87,35 @@ def k_contiguous_b(b: torch.Tensor, rows_a: int) -> torch.Tensor:
 
 
 # Rows of A from which the GEMM reads a K-contiguous copy of B although the vector loaders take
-# an N-contiguous B. The product gains 2-4 % and the copy costs as much: 16384 x 2048 x 11264
-# 508 + 14 us against 519; below, the copy only loses (8192 x 1280 x 6400 111 + 8 against 113,
-# 4096 x 1280 x 6400 75 + 7 against 74).
+# an N-contiguous B. The product gains 1-4 % from the copy, which costs as much there. Measured,
+# us, copy and product against direct, operands from HBM: below, 8192 x 1280 x 8960 172 / 166
+# and 8192 x 2048 x 11264 263 / 256; at 16384 rows 351 / 349 and 504 / 510; above, 24576 rows
+# 403 / 411 and 748 / 764, 32768 rows 576 / 594 and 996 / 1018. (The exception below is a long
+# reduction at few rows, where the copy also brings B into the caches: 4096 x 2048 x 11264
+# 180 / 204.)
 DIRECT_MAX_ROWS = 16384
 
 
-def gemm_b(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
+def _vector_rows(t: torch.Tensor) -> bool:
+    """Whether the rows of a matrix are whole aligned 16-byte pieces, as a vector loader reads
+    them."""
+    return (t.stride(1) == 1 and t.shape[1] % 8 == 0 and t.stride(0) % 8 == 0
+            and t.data_ptr() % 16 == 0)
+
+
+def gemm_b(a: torch.Tensor, b: torch.Tensor, vector_out: bool = True) -> torch.Tensor:
     """B [K, N] as the GEMM of ``a`` [M, K] reads it: ``k_contiguous_b``'s copy, or B itself
-    where the vector loaders read an N-contiguous B directly at no loss: below
-    ``DIRECT_MAX_ROWS`` rows, and beside a token-major A (a weight gradient's dY.T: both
-    operands go through the transposing reads). Same bits."""
-    m, n = a.shape[0], b.shape[1]
-    if b.stride(1) == 1 and n % 8 == 0 and b.stride(0) % 8 == 0 and b.data_ptr() % 16 == 0:
-        token_major = (a.stride(0) == 1 and m % 8 == 0 and a.stride(1) % 8 == 0
-                       and a.data_ptr() % 16 == 0)
-        if token_major or m < DIRECT_MAX_ROWS:
+    where the vector GEMM reads an N-contiguous B directly: below ``DIRECT_MAX_ROWS`` rows,
+    and beside a token-major A (a weight gradient's dY.T: both operands go through the
+    transposing reads). An A that the vector loaders refuse, or outputs that are not 16-byte
+    pieces (``vector_out``), leave the product to the generic kernel, which reads a
+    K-contiguous B 1.3-1.5 times as fast (4096 x 1280 x 4480 with an unaligned A: 559 us with
+    the copy, 824 without). Same bits."""
+    if vector_out and _vector_rows(b):
+        token_major = _vector_rows(a.T)
+        if token_major or (_vector_rows(a) and a.shape[0] < DIRECT_MAX_ROWS):
             return b
-    return k_contiguous_b(b, m)
+    return k_contiguous_b(b, a.shape[0])
 
 
 def mm(a: torch.Tensor, b: torch.Tensor, algorithm: str = "tiled", tile: int = 0) -> torch.Tensor:
@@ -253,7 +264,8 @@ def swiglu_backward_mm(grad: torch.Tensor, down_weight: torch.Tensor, packed: to
     if out is None:
         out = torch.empty((m, 2 * h), dtype=torch.bfloat16, device=grad.device)
     _check_buffer(out, (m, 2 * h), torch.bfloat16, grad.device, "out")
-    down_weight = gemm_b(grad, down_weight)
+    vector_out = packed.data_ptr() % 16 == 0 and out.data_ptr() % 16 == 0
+    down_weight = gemm_b(grad, down_weight, vector_out)
     _hip.call("ws_swiglu_backward_mm", grad.data_ptr(), grad.stride(0), grad.stride(1),
               down_weight.data_ptr(), down_weight.stride(0), down_weight.stride(1),
               packed.data_ptr(), out.data_ptr(), m, h, k, int(eager_rounding), _hip.stream(grad))
