@@ -25,7 +25,9 @@
  * `algorithm` (GEMM entry points): 0 = "tiled" (one workgroup per output tile),
  * 1 = "persistent" (one resident workgroup per CU slot striding over tiles),
  * 2 = "persistent_tma" (persistent, with the reference's TMA preconditions checked by the
- * caller). `tile`: 0 = 256x256 macro-tile (8 waves), 1 = 128x128 macro-tile (4 waves).
+ * caller). `tile`: 0 = the vector kernels' macro-tile for these sizes (256x256 to 64x64, see
+ * ws_gemm_tile; 256x256 with 8 waves for operands that the vector loaders refuse), 1 = the
+ * general kernel's 128x128 macro-tile (4 waves).
  *
  * Reference citations are path:line in gtausa197-svg/WarpState-AI.
  */
@@ -63,6 +65,27 @@ int ws_mm(const void* a, int64_t a_s0, int64_t a_s1, const void* b, int64_t b_s0
 int ws_swiglu_mm(const void* a, int64_t a_s0, int64_t a_s1, const void* b, int64_t b_s0,
                  int64_t b_s1, void* packed, void* act, int64_t m, int64_t h, int64_t k,
                  int eager_rounding, int algorithm, int tile, void* stream);
+
+/* The macro-tile that ws_mm, ws_swiglu_mm (tile 0), ws_residual_mm, ws_rmsnorm_gate_mm and
+ * ws_swiglu_backward_mm run an [m, n] output with reduction k on, for operands that the vector
+ * loaders take: 0 = 256 x 256, 1 = 128 x 128 (two workgroups per CU), 2 = 128 x 128 (one),
+ * 3 = 64 x 128, 4 = 64 x 64; -1 for invalid sizes. `n` is the packed width 2h of the paired
+ * SwiGLU projection and h of the SwiGLU backward. Operands: A [m, k] with k or (token-major)
+ * m contiguous, B [k, n] with k or n contiguous. Launches nothing. */
+enum WsEpilogue {
+  WS_EPI_STORE = 0,
+  WS_EPI_RESIDUAL = 1,
+  WS_EPI_SIGMOID = 2,
+  WS_EPI_SWIGLU = 3,
+  WS_EPI_SWIGLU_BACKWARD = 4
+};
+int ws_gemm_tile(int64_t m, int64_t n, int64_t k, int a_token_major, int b_n_contiguous,
+                 int epilogue);
+
+/* The same for one FP32 gradient (ws_mm_accumulate_f32, or ws_mm_store_f32 with `store`) of
+ * token-major operands whose caller allows `splits` k-slices; *slices (may be null) receives
+ * the slices of a smaller tile, or `splits` for 256 x 256 tiles. Launches nothing. */
+int ws_mm_f32_tile(int64_t m, int64_t n, int64_t k, int64_t splits, int store, int* slices);
 
 /* Standalone SwiGLU of a contiguous packed [rows, 2h] BF16 projection; replaces
  * bf16_swiglu (ops/activation_execution.py:58-70). */

@@ -1,16 +1,14 @@
-"""Bit-exact GPU checks of the 256 x 256 GEMM's four operand layouts at the k-tile counts
-its pipelines treat specially.
+"""Bit-exact GPU checks of small vector-operand products in all four operand layouts, at few
+k-tiles.
 
 Integer-valued BF16 operands in [-3, 3] make every FP32 partial sum an integer below 2^24,
 so any summation order gives the exact product, and the BF16 output must equal the
 exactly rounded product bit for bit (the reference's layout test,
 test_matmul_kernels.py:147-188, holds its kernels to a BF16 bar on random data; exact
 operands pin the fragment, stage and output indexing here). The shapes cover one to five
-64-wide k-tiles (with both operands K-contiguous, B runs through three LDS stages and its
-first two k-tiles are issued before the loop; with both M/N-contiguous, the next k-tile's
-loads are issued at the top of each k-tile), a ragged last k-tile, ragged row and column
-tiles, and a reduction long enough for the stages to wrap many times. Every width is a
-multiple of 8, so every operand takes a vector loader and the launch the 256 x 256 path.
+64-wide k-tiles, a ragged last k-tile, ragged row and column tiles, and a longer reduction.
+Every width is a multiple of 8, so every operand takes a vector loader. Outputs this small
+run on the 64 x 64 macro-tile; test_gpu_tiles.py holds every macro-tile to the same bar.
 """
 import pytest
 import torch

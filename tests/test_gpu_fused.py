@@ -30,9 +30,10 @@ def _gen(seed):
                                    (300, 272, 200), (520, 528, 1000)])
 @pytest.mark.parametrize("tile", [(64, 64, 32, 4, 3), (128, 128, 32, 8, 3)])
 def test_swiglu_projection_and_activation(algorithm, eager_rounding, shape, tile):
-    """(M, 2H, K). The last two shapes take the 256 x 256 paired kernel (K a multiple of 8)
-    with every edge ragged: partial row tiles, a half width H that is not a multiple of
-    the 128 columns a paired tile holds per half, and a partial last k-tile."""
+    """(M, 2H, K). The last two shapes take the vector loaders (K a multiple of 8) with every
+    edge ragged: partial row tiles, a half width H that is not a multiple of the 64 columns
+    a paired 64 x 128 tile holds per half, and a partial last k-tile. (test_gpu_tiles.py
+    covers the other macro-tiles.)"""
     from ops.matmul_epilogue import launch_swiglu_mm
 
     m, packed_width, k = shape

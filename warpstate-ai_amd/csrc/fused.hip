@@ -80,7 +80,7 @@ extern "C" int ws_rmsnorm_gate_mm(const void* x, int64_t x_s0, const float* norm
   p.gate_hi = (int)gate_end;
   int am = operand_mode(p.a, m, k, 256), bm = operand_mode(p.b, n, k, 256);
   if (fast_ok(p, am, bm, false))
-    return dispatch_tiles<kMaskKRows, false, FEpiStore<true, false>>(p, am, bm, kFusedCfg, s, kEpiSigmoid);
+    return dispatch_tiles<WS_EPI_SIGMOID, FEpiStore<true, false>>(p, am, bm, kFusedCfg, s);
   return dispatch<kMaskMM, WS_TILE_ARGS_LARGE, false, EpiStore<true, false>>(p, am, bm,
                                                                                    LaunchCfg{0, 1}, s);
 }
@@ -105,7 +105,7 @@ extern "C" int ws_residual_mm(const void* a, int64_t a_s0, int64_t a_s1, const v
   int am = operand_mode(p.a, m, k, 256), bm = operand_mode(p.b, n, k, 256);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (fast_ok(p, am, bm, false))
-    return dispatch_tiles<kMaskKRows, false, FEpiStore<false, true>>(p, am, bm, kFusedCfg, s);
+    return dispatch_tiles<WS_EPI_RESIDUAL, FEpiStore<false, true>>(p, am, bm, kFusedCfg, s);
   constexpr unsigned mask = kMaskKK | ab_bit(kKContig, kMNContig) | kMaskGG;
   return dispatch<mask, WS_TILE_ARGS_LARGE, false, EpiStore<false, true>>(
       p, am, bm, LaunchCfg{0, 1}, s);
@@ -132,7 +132,7 @@ extern "C" int ws_swiglu_backward_mm(const void* grad, int64_t g_s0, int64_t g_s
   int am = operand_mode(p.a, m, k, 256), bm = operand_mode(p.b, h, k, 256);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (fast_ok(p, am, bm, false))
-    return dispatch_tiles<kMaskKRows, false, FEpiSwigluBwd>(p, am, bm, kFusedCfg, s, kEpiSwigluBwd);
+    return dispatch_tiles<WS_EPI_SWIGLU_BACKWARD, FEpiSwigluBwd>(p, am, bm, kFusedCfg, s);
   constexpr unsigned mask = kMaskKK | ab_bit(kKContig, kMNContig) | kMaskGG;
   return dispatch<mask, WS_TILE_ARGS_LARGE, false, EpiSwigluBwd>(
       p, am, bm, LaunchCfg{0, 1}, s);
@@ -271,6 +271,14 @@ WgradPlan wgrad_plan(long m, long n, long k, int splits, bool store, int workers
 }
 
 }  // namespace
+
+extern "C" int ws_mm_f32_tile(int64_t m, int64_t n, int64_t k, int64_t splits, int store,
+                              int* slices) {
+  if (m < 1 || n < 1 || k < 1 || splits < 1 || splits > 64) return -1;
+  const WgradPlan plan = wgrad_plan(m, n, k, (int)splits, store != 0, device_cus());
+  if (slices) *slices = plan.splits;
+  return plan.tile;
+}
 
 extern "C" int64_t ws_mm_accumulate_workspace_floats(int64_t m, int64_t n, int64_t k, int64_t splits) {
   if (splits <= 1 || m < 1 || n < 1 || k < 1) return 0;

@@ -313,14 +313,30 @@ int run_ring_tile(const GemmParams& p, int tile, hipStream_t s, int splits = 1) 
   return set_error(kInvalid, "no GEMM macro-tile %d", tile);
 }
 
-// The fast path with the macro-tile picked by tile_time. MASK holds the operand layouts
+// The fast path with the macro-tile picked by tile_time. A rule's mask holds the operand layouts
 // (ab_bit) the smaller tiles are built for; the others run on 256 x 256 tiles.
 constexpr unsigned kMaskKRows = ab_bit(kKContig, kKContig) | ab_bit(kKContig, kMNContig);
 constexpr unsigned kMaskVector = kMaskKRows | ab_bit(kMNContig, kKContig) | ab_bit(kMNContig, kMNContig);
-template <unsigned MASK, bool PAIRED, class Epi>
-int dispatch_tiles(const GemmParams& p, int am, int bm, LaunchCfg cfg, hipStream_t s,
-                   float epi = kEpiStore) {
-  const int tile = (MASK & ab_bit(am, bm)) ? pick_tile(p.M, p.N, p.K, am, bm, PAIRED, epi) : kTile256;
+struct TileRule {
+  unsigned mask;
+  bool paired;
+  EpiCost epi;
+};
+// By WsEpilogue (include/warpstate_hip.h).
+constexpr TileRule kTileRules[] = {{kMaskVector, false, kEpiStore},
+                                   {kMaskKRows, false, kEpiStore},
+                                   {kMaskKRows, false, kEpiSigmoid},
+                                   {kMaskKRows, true, kEpiSwiglu},
+                                   {kMaskKRows, false, kEpiSwigluBwd}};
+inline int rule_tile(const TileRule& r, long m, long n, long k, int am, int bm) {
+  return (r.mask & ab_bit(am, bm)) ? pick_tile(m, n, k, am, bm, r.paired, r.epi) : kTile256;
+}
+
+template <int RULE, class Epi>
+int dispatch_tiles(const GemmParams& p, int am, int bm, LaunchCfg cfg, hipStream_t s) {
+  constexpr unsigned MASK = kTileRules[RULE].mask;
+  constexpr bool PAIRED = kTileRules[RULE].paired;
+  const int tile = rule_tile(kTileRules[RULE], p.M, p.N, p.K, am, bm);
   if (tile == kTile256) return dispatch_fast<PAIRED, Epi>(p, am, bm, cfg, s);
 #define WS_RING(A_, B_)                                                          \
   if constexpr ((MASK & ab_bit(A_, B_)) != 0)                                    \

@@ -52,7 +52,7 @@ extern "C" int ws_mm(const void* a, int64_t a_s0, int64_t a_s1, const void* b, i
   LaunchCfg cfg{algorithm != 0, 1};
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (tile == kTileLarge && fast_ok(p, am, bm, false))
-    return dispatch_tiles<kMaskVector, false, FEpiStore<false, false>>(p, am, bm, cfg, s);
+    return dispatch_tiles<WS_EPI_STORE, FEpiStore<false, false>>(p, am, bm, cfg, s);
   if (tile == kTileLarge)
     return dispatch<kMaskMM, WS_TILE_ARGS_LARGE, false, EpiStore<false, false>>(p, am, bm, cfg, s);
   return dispatch<kMaskMM, WS_TILE_ARGS_SMALL, false, EpiStore<false, false>>(p, am, bm, cfg, s);
@@ -88,8 +88,17 @@ extern "C" int ws_swiglu_mm(const void* a, int64_t a_s0, int64_t a_s1, const voi
   LaunchCfg cfg{algorithm != 0, 1};
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (tile == kTileLarge && fast_ok(p, am, bm, true))
-    return dispatch_tiles<kMaskKRows, true, FEpiSwiglu>(p, am, bm, cfg, s, kEpiSwiglu);
+    return dispatch_tiles<WS_EPI_SWIGLU, FEpiSwiglu>(p, am, bm, cfg, s);
   if (tile == kTileLarge)
     return dispatch<kMaskKK | kMaskGG, WS_TILE_ARGS_LARGE, true, EpiSwiglu>(p, am, bm, cfg, s);
   return dispatch<kMaskKK | kMaskGG, WS_TILE_ARGS_SMALL, true, EpiSwiglu>(p, am, bm, cfg, s);
+}
+
+extern "C" int ws_gemm_tile(int64_t m, int64_t n, int64_t k, int a_token_major, int b_n_contiguous,
+                            int epilogue) {
+  if (m < 1 || n < 1 || k < 1 || epilogue < 0 ||
+      epilogue >= (int)(sizeof(kTileRules) / sizeof(kTileRules[0])))
+    return -1;
+  return rule_tile(kTileRules[epilogue], m, n, k, a_token_major ? kMNContig : kKContig,
+                   b_n_contiguous ? kMNContig : kKContig);
 }

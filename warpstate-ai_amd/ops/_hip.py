@@ -30,6 +30,8 @@ SIGNATURES = {
                      _i32, _i32, _c_void_p]),
     "ws_swiglu_mm": (_i32, [_c_void_p, _i64, _i64, _c_void_p, _i64, _i64, _c_void_p, _c_void_p,
                             _i64, _i64, _i64, _i32, _i32, _i32, _c_void_p]),
+    "ws_gemm_tile": (_i32, [_i64, _i64, _i64, _i32, _i32, _i32]),
+    "ws_mm_f32_tile": (_i32, [_i64, _i64, _i64, _i64, _i32, _c_void_p]),
     "ws_swiglu_forward": (_i32, [_c_void_p, _c_void_p, _i64, _i64, _i32, _c_void_p]),
     "ws_swiglu_backward": (_i32, [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i32, _c_void_p]),
     "ws_rmsnorm_forward": (_i32, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _f32,
@@ -170,9 +172,10 @@ def algorithm_code(algorithm: str) -> int:
 
 
 def tile_code(block_m: int, block_n: int) -> int:
-    """Macro-tile for a requested (block_m, block_n): 0 = 256x256, 1 = 128x128.
+    """`tile` argument for a requested (block_m, block_n).
 
-    Requests of at least 128x128 outputs use the 256x256 8-wave tile; smaller requests
-    use the 128x128 4-wave tile that keeps two workgroups per CU.
+    Requests of at least 128x128 outputs (0) take the vector kernels, whose macro-tile
+    follows the sizes (``ws_gemm_tile``); smaller requests (1) the general kernel's 128x128
+    4-wave tile, two workgroups per CU.
     """
     return 0 if block_m * block_n >= 128 * 128 else 1

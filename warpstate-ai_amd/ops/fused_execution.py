@@ -119,7 +119,8 @@ def gemm_b(a: torch.Tensor, b: torch.Tensor, vector_out: bool = True) -> torch.T
 
 
 def mm(a: torch.Tensor, b: torch.Tensor, algorithm: str = "tiled", tile: int = 0) -> torch.Tensor:
-    """r(a @ b) with the HIP GEMM; `tile` 0 = 256x256, 1 = 128x128."""
+    """r(a @ b) with the HIP GEMM; `tile` 0 = the macro-tile for the sizes, 1 = the general
+    kernel's 128x128 (``_hip.tile_code``)."""
     _check_bf16_cuda(a, b)
     if a.ndim != 2 or b.ndim != 2 or a.shape[1] != b.shape[0]:
         raise ValueError(f"Expected a [M, K] and b [K, N], got {list(a.shape)} and {list(b.shape)}")
