@@ -1,14 +1,15 @@
-"""Static check of the inline-assembly transposing reads in the 256 x 256 GEMM (CPU only).
+"""Static check of the inline-assembly fragment reads in the 256 x 256 GEMM (CPU only).
 
-With both operands M/N-contiguous, the k-loop issues its fragment reads as inline
-assembly (``ds_read_b64_tr_b16``), which the compiler does not know to be LDS loads: it
-inserts no wait before their results are used. Their results become usable only at the
-explicit ``s_waitcnt lgkmcnt(0)`` that follows them (``tie_wait``). Until then no
-instruction may read or write a destination register of a pending read, and no branch may
-leave with one pending. The GPU tests check the results; this test compiles the kernels
+The k-loop issues all of its fragment reads as inline assembly (``ds_read_b64_tr_b16`` of an
+M/N-contiguous operand, ``ds_read_b128`` of a K-contiguous one), which the compiler does not
+know to be LDS loads: it inserts no wait before their results are used. Their results become
+usable only at the explicit ``s_waitcnt lgkmcnt(0)`` that follows them (``tie_wait``). Until
+then no instruction may read or write a destination register of a pending read, and no branch
+may leave with one pending. The GPU tests check the results; this test compiles the kernels
 to gfx950 assembly with the library's build flags and checks that rule on every
-instantiation that uses the assembly reads, so that a compiler that moves or copies a
-fragment register ahead of its wait fails here, before any GPU run.
+instantiation, so that a compiler that moves or copies a fragment register ahead of its wait
+fails here, before any GPU run. (The epilogues' own LDS reads go through the compiler, which
+waits for them itself, with counted waits that this check does not model.)
 """
 import re
 import shutil
@@ -41,52 +42,67 @@ def _regs(operands: str) -> set[int]:
     return out
 
 
+_compiled: dict[str, str] = {}  # by source, for this module and test_asm_hazards_ring.py
+
+
 def _assembly(source: str, tmp_path: Path) -> str:
+    if source in _compiled:
+        return _compiled[source]
     target = tmp_path / (Path(source).stem + ".s")
     cmd = [HIPCC, *build_lib.FLAGS, f"-I{build_lib.CSRC}", "--cuda-device-only", "-S",
            str(build_lib.CSRC / source), "-o", str(target)]
     result = subprocess.run(cmd, capture_output=True, text=True)
     assert result.returncode == 0, result.stderr[-2000:]
-    return target.read_text()
+    _compiled[source] = target.read_text()
+    return _compiled[source]
 
 
 def _kernels(text: str) -> dict[str, list[str]]:
-    """Bodies of the unpaired gemm_fast_kernel<1, 1, false, ...> instantiations (both
-    operands M/N-contiguous), the ones whose k-loop uses the assembly reads. The paired
-    instantiation reads through the compiler's builtin, which the compiler waits for itself
-    with counted waits that this check does not model."""
+    """Bodies of the gemm_fast_kernel<AMODE, BMODE, PAIRED, ...> instantiations."""
     bodies, name = {}, None
     for line in text.splitlines():
-        m = re.match(r"^(_ZN2ws16gemm_fast_kernelILi1ELi1ELb0E\w*):", line)
+        m = re.match(r"^(_ZN2ws16gemm_fast_kernelILi[01]ELi[01]ELb[01]E\w*):", line)
         if m:
             name = m.group(1)
             bodies[name] = []
         elif name is not None:
-            if line.strip().startswith("s_endpgm"):
+            if line.startswith(".Lfunc_end"):
                 name = None
             else:
                 bodies[name].append(line)
     return bodies
 
 
+def _assembly_reads(body: list[str]) -> list[tuple[str, bool]]:
+    """(instruction, whether it stands in inline assembly), comments and labels dropped."""
+    out, inside = [], False
+    for raw in body:
+        text = raw.strip()
+        if text.startswith((";;#ASMSTART", ";;#ASMEND")):
+            inside = "START" in text
+            continue
+        line = text.split(";")[0].strip()
+        if line and not line.endswith(":") and not line.startswith("."):
+            out.append((line, inside))
+    return out
+
+
 def _violations(body: list[str]) -> tuple[int, list[str]]:
     pending: set[int] = set()
     reads, bad = 0, []
-    for raw in body:
-        line = raw.split(";")[0].strip()
-        if not line or line.endswith(":") or line.startswith("."):
-            continue
+    for line, assembly in _assembly_reads(body):
         mnemonic, _, operands = line.partition(" ")
         if mnemonic == "s_waitcnt":
             if "lgkmcnt(0)" in operands:
                 pending.clear()
             continue
         used = _regs(operands)
-        if mnemonic == TR_READ:
+        if mnemonic == TR_READ or (assembly and mnemonic == "ds_read_b128"):
             reads += 1
             dest = _regs(operands.split(",")[0])
-            if dest & pending:
-                bad.append(f"overwrites a pending read's register: {line}")
+            # A second read into a pending register, or an address taken from one.
+            if used & pending:
+                bad.append(f"touches a pending read's register: {line}")
             pending |= dest
             continue
         if pending and mnemonic.startswith(("s_branch", "s_cbranch", "s_setpc", "s_swappc")):
@@ -98,13 +114,19 @@ def _violations(body: list[str]) -> tuple[int, list[str]]:
     return reads, bad
 
 
-@pytest.mark.parametrize("source", ["mm.hip", "fused.hip"])
-def test_transposing_reads_are_waited_for_before_use(source, tmp_path):
+# Instantiations per source: four operand layouts for every epilogue that runs there, the
+# paired one (mm.hip) included.
+@pytest.mark.parametrize("source,count", [("mm.hip", 8), ("fused.hip", 20), ("ce.hip", 24)])
+def test_fragment_reads_are_waited_for_before_use(source, count, tmp_path):
     kernels = _kernels(_assembly(source, tmp_path))
-    checked = {name: _violations(body) for name, body in kernels.items()}
-    assert checked, f"no unpaired M/N-contiguous instantiation in {source}"
-    for name, (reads, bad) in checked.items():
-        assert reads >= 48, (name, reads)  # 24 reads per k32 step, two steps per k-tile
+    assert len(kernels) == count, (source, sorted(kernels))
+    for name, body in kernels.items():
+        a_mn, b_mn = re.match(r".*?ILi(\d)ELi(\d)E", name).groups()
+        # A k-tile's two k32 steps read 4 A and 8 B blocks each, a transposed block in two
+        # reads.
+        per_tile = 2 * (4 * (1 + int(a_mn)) + 8 * (1 + int(b_mn)))
+        reads, bad = _violations(body)
+        assert reads >= per_tile and reads % per_tile == 0, (name, reads, per_tile)
         assert not bad, (name, bad[:5])
 
 
@@ -121,3 +143,8 @@ def test_checker_flags_a_use_before_the_wait():
     assert _violations([read, "\ts_cbranch_scc1 .LBB0_5", wait])[1]
     assert _violations([read, "\tv_add_u32_e32 v30, v31, v32", wait]) == (1, [])
     assert _violations([read])[1]
+    rows = [";;#ASMSTART", "\tds_read_b128 v[20:23], v201", ";;#ASMEND"]
+    assert _violations([*rows, wait, mfma]) == (1, [])
+    assert _violations([*rows, mfma, wait])[1]
+    assert _violations([*rows, read, wait]) == (2, [])
+    assert _violations([rows[1], mfma]) == (0, [])  # the compiler's own read
