@@ -35,7 +35,13 @@
 //    groups have read it. The 8 waves in step on one barrier per k-tile left the matrix pipe
 //    idle while all of them read their first fragments; one box, alternated, same bits, us:
 //    16384 x 9216 x 2048 460 -> 436, 16384 x 2048 x 11264 536 -> 501, 8192 x 8192 x 8192
-//    772 -> 717 (1.53 PFLOP/s), 16384 x 2048 x 5632 275 -> 257. Moving B's second-step reads
+//    772 -> 717 (1.53 PFLOP/s), 16384 x 2048 x 5632 275 -> 257. The last two k-tiles load
+//    nothing ahead. (Zero-filling loads there kept the waits' counts, but the epilogue waited
+//    for them, and a piece that ended before K fetched the next piece's operands: one box,
+//    alternated, us, before / now: 4096 x 3072 x 64 10.1 / 9.4, token-major A 10.7 / 9.5,
+//    4096 x 3072 x 512 17.9 / 17.4, 16384 x 2048 x 11264 501 / 488, the balanced 9216 x 2048
+//    gradient over 16384 tokens 491 / 478; the same guard as a branch in the one loop made an
+//    N-contiguous B 2 % slower instead.) Moving B's second-step reads
 //    into the MFMA phase, s_setprio around it and the loads between the reads change nothing:
 //    the clock gives way (32x32x16 MFMAs: 11 % slower).
 //  * The fragment reads are inline assembly with explicit lgkmcnt waits: the compiler orders
@@ -832,8 +838,8 @@ __global__ void __launch_bounds__(kFNT) gemm_fast_kernel(const GemmParams p) {
 #pragma unroll
           for (int i = 0; i < kFIns; ++i) dma16(rs, dst + i * 4096, off[i]);
         } else {
-          // Ragged or past the end: chunks at k >= K land as zeros. The lane index goes
-          // through an empty asm so that the k offsets are not kept live across the loop.
+          // Ragged: chunks at k >= K land as zeros. The lane index goes through an empty asm
+          // so that the k offsets are not kept live across the loop.
           int l = lane;
           asm volatile("" : "+v"(l));
 #pragma unroll
@@ -848,28 +854,38 @@ __global__ void __launch_bounds__(kFNT) gemm_fast_kernel(const GemmParams p) {
         __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
       } else {
         load(kb, sB);
-        load(kb + 1, sB + kFTileBytes);
-        __builtin_amdgcn_s_waitcnt(wait_vmcnt(kFIns));  // B(kb)
+        if (kb + 1 < ke) {
+          load(kb + 1, sB + kFTileBytes);
+          __builtin_amdgcn_s_waitcnt(wait_vmcnt(kFIns));  // B(kb)
+        } else {
+          __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
+        }
       }
       __builtin_amdgcn_s_barrier();
       if (!first) __builtin_amdgcn_s_barrier();  // one phase behind from here on
       unsigned ast = 0, bst = 0;  // byte offsets of the k-tile's stages
-      for (int kt = kb; kt < ke; ++kt) {
+      // k-tile kt; the last two (TAIL) load nothing past the piece: those loads would fetch
+      // another slice's operands or zeros, and the epilogue would wait for them.
+      auto k_tile = [&](int kt, auto tail) {
+        constexpr bool TAIL = decltype(tail)::value;
         // Read phase. A(kt + 1) goes to the stage A(kt - 1) used and B(kt + 2) to the one
-        // B(kt - 1) used: both groups have read those. Loads past the last k-tile land as
-        // zeros and keep the counts.
-        load(first ? kt + 1 : kt + 2,
-             first ? sA + (ast ^ kFTileBytes) : sB + (bst == 0 ? 2 * kFTileBytes : bst - kFTileBytes));
+        // B(kt - 1) used: both groups have read those.
+        if (!TAIL)
+          load(first ? kt + 1 : kt + 2,
+               first ? sA + (ast ^ kFTileBytes) : sB + (bst == 0 ? 2 * kFTileBytes : bst - kFTileBytes));
+        else if (first && kt + 1 < ke)
+          load(kt + 1, sA + (ast ^ kFTileBytes));
         __builtin_amdgcn_sched_barrier(0);
         bf16x8_t f[2 * (FA + FB)];
         asm_frags<AMODE, BMODE, PAIRED, 0>(f, abase + ast, bbase + bst);
         __builtin_amdgcn_sched_barrier(0);
         // B(kt + 1) has landed (only the second group has older loads in flight here).
-        __builtin_amdgcn_s_waitcnt(wait_vmcnt(kFIns));
+        if (!TAIL) __builtin_amdgcn_s_waitcnt(wait_vmcnt(kFIns));
         tie_wait(f);
         __builtin_amdgcn_sched_barrier(0);
-        // Before the first group's epilogue stages through LDS: no load may be in flight.
-        if (kt + 1 == ke) __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
+        // In the last k-tile neither group has a load in flight from here on, so that the
+        // first group's epilogue may stage through LDS.
+        if (TAIL && !first) __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         // MFMA phase.
@@ -884,11 +900,14 @@ __global__ void __launch_bounds__(kFNT) gemm_fast_kernel(const GemmParams p) {
         __builtin_amdgcn_sched_barrier(0);
         if (first) __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));  // A(kt + 1) has landed
         // The second group's last MFMA phase ends the loop: the first group is past it.
-        if (first || kt + 1 < ke) __builtin_amdgcn_s_barrier();
+        if (!TAIL || first || kt + 1 < ke) __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         ast ^= kFTileBytes;
         bst = bst == 2 * kFTileBytes ? 0 : bst + kFTileBytes;
-      }
+      };
+      int kt = kb;
+      for (; kt + 2 < ke; ++kt) k_tile(kt, std::false_type{});
+      for (; kt < ke; ++kt) k_tile(kt, std::true_type{});
     }
     const int m_base = row0_a + wm * TM;
     const int n_base = row0_b + (PAIRED ? wn * (TN / 2) : wn * TN);

@@ -113,6 +113,11 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_ring_kernel(const GemmParams p) 
   const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
   const int kb = blockIdx.y * p.k_tiles_per_split;
   const int ke = min(cdiv(p.K, kFBK), kb + p.k_tiles_per_split);
+  // The loads ahead of the loop end with the piece: past it they fetch nothing and land as
+  // zeros, which keeps the count that the waits rely on. (The k-slices' epilogue alone runs
+  // on pieces that end before K.)
+  constexpr bool kSlices = std::is_same<Epi, FEpiAccF32<true>>::value;
+  const int k_end = kSlices ? min(p.K, ke * kFBK) : p.K;
 
   int tm, tn;
   tile_position(xcd_remap(blockIdx.x, p.total_tiles, kRingWindow), p.tiles_m, p.tiles_n, tm, tn);
@@ -142,8 +147,8 @@ __global__ void __launch_bounds__(Cfg::NT) gemm_ring_kernel(const GemmParams p) 
 
   auto issue = [&](int kt, int stage) {
     unsigned char* st = rsmem + stage * Cfg::kStage;
-    la.issue(p.a, row0_a, kt * kFBK, p.K, st, wave, lane);
-    lb.issue(p.b, row0_b, kt * kFBK, p.K, st + Cfg::kTileA, wave, lane);
+    la.issue(p.a, row0_a, kt * kFBK, k_end, st, wave, lane);
+    lb.issue(p.b, row0_b, kt * kFBK, k_end, st + Cfg::kTileA, wave, lane);
   };
   if (kb < ke) {
 #pragma unroll
