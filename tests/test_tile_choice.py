@@ -1,5 +1,7 @@
 """Every macro-tile of the GEMM dispatch stays within reach of the GPU tests' shapes (CPU only;
 the queries answer for 256 compute units where there is no GPU)."""
+import ctypes
+
 import pytest
 
 from ops import _hip
@@ -35,6 +37,18 @@ def test_each_gradient_tile_is_reached(store):
         assert gradient_shape(tile, 1, 1, store, 8200)
         for splits in (2, 4):
             assert gradient_shape(tile, splits, splits, store, 8200), (tile, splits)
+
+
+# Gradients whose last round on a smaller tile holds a pair on a few compute units only, with
+# the time of that tile and of the 256 x 256 schemes, us.
+@pytest.mark.parametrize("m,n,k,splits,store,slow,us", [
+    (1400, 1632, 6601, 4, 0, (3, 1), (79, 59)), (592, 3816, 5622, 4, 0, (3, 1), (72, 47)),
+    (3184, 856, 4363, 4, 1, (3, 1), (55, 45)), (4376, 1048, 8414, 2, 1, (1, 1), (121, 107)),
+    (6312, 680, 8448, 2, 1, (1, 1), (123, 106))])
+def test_a_few_pairs_do_not_end_the_launch_late(m, n, k, splits, store, slow, us):
+    got = ctypes.c_int()
+    tile = _hip.query("ws_mm_f32_tile", m, n, k, splits, store, ctypes.byref(got))
+    assert (tile, got.value) != slow
 
 
 def test_invalid_sizes():

@@ -241,16 +241,24 @@ float balanced_time(const BalancedPlan& b, bool store, int workers) {
   return loop + rounds +
          (b.sk_tiles ? 4.0f + 4.0f * kFBM * kFBN * (float)b.sk_tiles * (b.pieces + 2) / 5.5e6f : 0.0f);
 }
+// us per k-tile of a token-major gradient's last round where some CUs hold a pair, however few:
+// the launch ends with theirs. By tile (launch.h), rows on whole 128-byte lines and off them,
+// where each row piece of a k-tile spans two lines (means over 1100 measured launches of 24
+// k-tiles or more; a lone workgroup 0.59, 0.35 and 0.26 in either case).
+constexpr float kSomePairs[kFastTiles][2] = {{0, 0}, {0.80f, 0.95f}, {0, 0}, {0.57f, 0.76f}, {0.40f, 0.55f}};
+
 // The cheapest way for a token-major gradient (both operands M/N-contiguous) whose caller
 // allows up to `splits` slices. The 256 x 256 schemes stay unless a smaller tile promises
-// 10 % more. Measured, us: 6400 x 1280 x 4096 66 + 20 (two slices and their sum)
+// 10 % more and, with kSomePairs, at most 3 % less (1400 x 1632 over 6601 tokens, 286 tiles of
+// 64 x 128: 79 us, 256 x 256 slices and their sum 59; 592 x 3816 x 5622 72 / 47, 6312 x 680 x
+// 8448 in two slices 123 / 106). Measured, us: 6400 x 1280 x 4096 66 + 20 (two slices and their sum)
 // against 68 (128 x 128); 1280 x 4480 + 8960 x 1280 over 512 tokens 40 + 6 (balanced, one
 // launch) against 16 + 23; over 1999 tokens 85 + 13 against 36 + 56 (balanced kept).
 WgradPlan wgrad_plan(long m, long n, long k, int splits, bool store, int workers) {
   const BalancedPlan b = balanced_plan(m, n, k, workers);
-  auto time = [&](int tile, int s) {
+  auto time = [&](int tile, int s, float some_pairs = 0.0f) {
     const float epi = s > 1 || store ? kEpiF32 : kEpiF32Add;
-    return tile_time(tile, m, n, k, kMNContig, kMNContig, workers, false, epi, s) +
+    return tile_time(tile, m, n, k, kMNContig, kMNContig, workers, false, epi, s, some_pairs) +
            (s > 1 ? reduce_time(m, n, s, store) : 0.0f);
   };
   WgradPlan best{kTile256, splits, 0.0f};
@@ -258,11 +266,13 @@ WgradPlan wgrad_plan(long m, long n, long k, int splits, bool store, int workers
     best.time = balanced_time(b, store, workers);
   else
     best.time = time(kTile256, b.sk_tiles == 0 ? 1 : splits);
-  float limit = 0.9f * best.time;
+  const float whole = best.time;
+  const bool off_lines = m % kFBK != 0 || n % kFBK != 0;
+  float limit = 0.9f * whole;
   for (int tile = kTile256 + 1; tile < kFastTiles; ++tile)
     for (int s = 1; s <= splits; ++s) {
       const float t = time(tile, s);
-      if (t < limit) {
+      if (t < limit && time(tile, s, kSomePairs[tile][off_lines]) < 1.03f * whole) {
         best = WgradPlan{tile, s, t};
         limit = t;
       }

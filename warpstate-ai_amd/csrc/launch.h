@@ -237,9 +237,10 @@ inline const TileCost& tile_cost(int tile, int am, int bm) {
 enum EpiCost { kEpiStore = 0, kEpiSigmoid = 2, kEpiSwiglu = 4, kEpiF32 = 6, kEpiF32Add = 18, kEpiSwigluBwd = 20 };
 
 // An [m, n] output (n the packed width of a paired GEMM) with reduction k in `copies` split-K
-// slices.
+// slices. A last round in which only some CUs hold a pair is priced between a lone workgroup's
+// time and a pair's, or with `some_pairs` us per k-tile.
 inline float tile_time(int tile, long m, long n, long k, int am, int bm, int cus, bool paired,
-                       float epi, long copies = 1) {
+                       float epi, long copies = 1, float some_pairs = 0.0f) {
   const TileCost& c = tile_cost(tile, am, bm);
   const long tiles = (long)cdiv(m, c.bm) * cdiv(n, c.bn) * copies;
   const float kt = (float)cdiv(cdiv(k, kFBK), copies), area = (float)(c.bm * c.bn) / 65536.0f;
@@ -256,7 +257,7 @@ inline float tile_time(int tile, long m, long n, long k, int am, int bm, int cus
   }
   const long rounds = tiles / (2 * cus), rest = tiles % (2 * cus);
   const float around = fixed + epi * area * 1.8f;
-  float pair = c.pair * slow;
+  const float pair = c.pair * slow > some_pairs ? c.pair * slow : some_pairs;
   float drift = 0.0f;
   if (tiles > 2 * cus) {
     drift = -c.settle + c.drift * (kt - 32.0f);
@@ -264,7 +265,8 @@ inline float tile_time(int tile, long m, long n, long k, int am, int bm, int cus
   }
   float t = (float)rounds * ((pair + drift) * kt + around);
   if (rest > cus)  // some CUs hold a pair
-    t += (alone + (pair - alone) * (float)(rest - cus) / (float)cus) * kt + around;
+    t += (some_pairs > 0.0f ? some_pairs : alone + (pair - alone) * (float)(rest - cus) / (float)cus) * kt +
+         around;
   else if (rest)
     t += alone * kt + fixed + epi * area;
   return t;
