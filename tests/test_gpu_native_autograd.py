@@ -121,7 +121,9 @@ def test_compiled_autograd_traces_the_native_nodes(name):
 
     torch._dynamo.reset()
     try:
-        grad = torch.randn_like(call(*leaves))
+        out = call(*leaves)
+        assert "Generated" not in out.grad_fn.name()  # the C++ node, not the Python formula's
+        grad = torch.randn_like(out)
         want = gradients(call, grad)
         for fn in (call, torch.compile(call, backend="aot_eager", fullgraph=True)):
             with compiled_autograd._enable(torch.compile(backend="aot_eager")):

@@ -73,13 +73,14 @@ def build(jobs: int | None = None) -> Path:
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         autograd = pool.submit(_build_autograd)
         objects = list(pool.map(_compile, sources))
-        autograd.result()
     staging = LIBRARY.with_name(LIBRARY.name + ".tmp")
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-o", str(staging), *map(str, objects)]
     result = subprocess.run(cmd, capture_output=True, text=True)
     if result.returncode != 0:
         raise RuntimeError("link failed:\n" + result.stderr)
     os.replace(staging, LIBRARY)
+    # Last, so that a host without PyTorch's headers is left with the kernels.
+    autograd.result()
     return LIBRARY
 
 

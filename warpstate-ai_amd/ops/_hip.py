@@ -3,13 +3,15 @@
 Every call passes raw device pointers, element strides and sizes, and the HIP stream of
 PyTorch's current stream on the calling thread. A non-zero status becomes a
 ``RuntimeError`` carrying the library's message. There is no fallback: when the library
-is missing, every kernel entry point raises.
+is missing, every kernel entry point raises. (The operators' C++ autograd nodes, a library of
+their own, do have one: ``load_autograd``.)
 """
 
 from __future__ import annotations
 
 import ctypes
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -129,16 +131,21 @@ _autograd_loaded = False
 
 def load_autograd() -> None:
     """Register the native autograd kernels of the row and fused training operators on CUDA
-    (``csrc/autograd.cpp``), once; raise if the kernels are built and these are not. Before
-    anything is built the operators import with their Python autograd formulas."""
+    (``csrc/autograd.cpp``), once. Without them (nothing built yet, the kernels alone built, or
+    a library of another PyTorch) the operators record their Python autograd formulas, which
+    give the same gradients for more host time; where the kernels are built, that is warned
+    about."""
     global _autograd_loaded
     with _lock:
         if _autograd_loaded or not LIBRARY_PATH.exists():
             return
-        if not AUTOGRAD_PATH.exists():
-            raise RuntimeError(f"native autograd kernels not built: {AUTOGRAD_PATH} is missing "
-                               "(run __graft_entry__.build())")
-        torch.ops.load_library(str(AUTOGRAD_PATH))
+        try:
+            torch.ops.load_library(str(AUTOGRAD_PATH))
+        except OSError as error:
+            warnings.warn(f"native autograd kernels not loaded ({error}); the operators use their "
+                          "Python autograd formulas (run __graft_entry__.build())",
+                          RuntimeWarning, stacklevel=2)
+            return
         _autograd_loaded = True
 
 
