@@ -251,9 +251,9 @@ constexpr float kSomePairs[kFastTiles][2] = {{0, 0}, {0.80f, 0.95f}, {0, 0}, {0.
 // allows up to `splits` slices. The 256 x 256 schemes stay unless a smaller tile promises
 // 10 % more and, with kSomePairs, at most 3 % less (1400 x 1632 over 6601 tokens, 286 tiles of
 // 64 x 128: 79 us, 256 x 256 slices and their sum 59; 592 x 3816 x 5622 72 / 47, 6312 x 680 x
-// 8448 in two slices 123 / 106). Measured, us: 6400 x 1280 x 4096 66 + 20 (two slices and their sum)
-// against 68 (128 x 128); 1280 x 4480 + 8960 x 1280 over 512 tokens 40 + 6 (balanced, one
-// launch) against 16 + 23; over 1999 tokens 85 + 13 against 36 + 56 (balanced kept).
+// 8448 in two slices 123 / 106). Measured, us, the 256 x 256 schemes against 128 x 128 tiles:
+// 6400 x 1280 over 4096 tokens 76 / 64; 1280 x 4480 and 8960 x 1280 over 512 tokens 44
+// (balanced, one launch) / 15 + 24, over 1999 tokens 92 / 32 + 57 (balanced kept).
 WgradPlan wgrad_plan(long m, long n, long k, int splits, bool store, int workers) {
   const BalancedPlan b = balanced_plan(m, n, k, workers);
   auto time = [&](int tile, int s, float some_pairs = 0.0f) {

@@ -188,16 +188,17 @@ enum FastTile { kTile256 = 0, kTile128x2, kTile128x1, kTile64x128, kTile64, kFas
 
 // Cost of one launch of each macro-tile in microseconds, fitted to sweeps of 150 shapes and
 // epilogues (128 to 16384 rows, 512 to 32768 columns, K 512 to 16384; outputs of all tiles the
-// same bits; the picks are within 2 % of the best tile in the geometric mean). A CU runs its
-// workgroups in rounds of one (`pair` 0) or two at a time; a round takes `alone` us per
+// same bits). Over 1600 others (128 to 16384 rows, 256 to 16384 columns, K 128 to 16384) the
+// picks are 1.3 to 3.3 % behind the best tile in the mean, by layout, and at most 47 %. A CU
+// runs its workgroups in rounds of one (`pair` 0) or two at a time; a round takes `alone` us per
 // 64-deep k-tile for one workgroup, `pair` us for two that share the CU, and `fixed` us
 // around the k-loop. The 256 x 256 tile costs less per product with every CU busy; below about
 // one round of its tiles most CUs idle, and a smaller tile wins although it loads its operands
-// more often. Measured, us (256 x 256 against the choice): 1999 x 1280 x 8960 136 / 71 (128 x
-// 128 alone), 4096 x 2048 x 5632 95 / 78 (128 x 128 paired), 1999 x 8960 x 1280 59 / 53; with
-// the 256 x 256 tile's former loop, 4-14 % slower: 512 x 1280 x 8960 159 / 40 (64 x 64), 128 x
-// 4800 x 960 23 / 7.4 (64 x 64); and where it stays: 8192 x 10240 x 2048 245 / 298, 8192 x
-// 2048 x 2048 51 / 59 (the best smaller tile).
+// more often. Measured, us (256 x 256 against the choice): 512 x 1280 x 8960 130 / 41 (64 x 64),
+// 1999 x 1280 x 8960 131 / 78 (64 x 128; 128 x 128 alone would take 73), 4096 x 2048 x 5632
+// 98 / 78 and 4096 x 1280 x 6400 102 / 72 (128 x 128 paired), 128 x 4800 x 960 20 / 7.5
+// (64 x 64); and where it stays: 1999 x 8960 x 1280 56 / 55, 8192 x 10240 x 2048 238 / 294,
+// 8192 x 2048 x 2048 51 / 60 (the best smaller tile).
 struct TileCost {
   int bm, bn;
   float alone, pair, fixed;  // pair 0: one workgroup per CU
@@ -232,7 +233,7 @@ inline const TileCost& tile_cost(int tile, int am, int bm) {
 }
 // What an epilogue costs beside a plain BF16 store, us per round of 256 x 256 tiles (every CU
 // in it at once, bound by HBM): the SwiGLU backward reads and writes the packed projection,
-// 8192 x 4096 x 1024 102 us against 58. A smaller tile's round pays by its area; two
+// 8192 x 4096 x 1024 97 us against 56. A smaller tile's round pays by its area; two
 // workgroups on a CU hide a tenth of it behind each other's k-loop.
 enum EpiCost { kEpiStore = 0, kEpiSigmoid = 2, kEpiSwiglu = 4, kEpiF32 = 6, kEpiF32Add = 18, kEpiSwigluBwd = 20 };
 

@@ -185,7 +185,9 @@ def rmsnorm_gate_mm(x: torch.Tensor, norm_weight: torch.Tensor, eps: float,
     if normed is None:
         normed = torch.empty((m, k), dtype=torch.bfloat16, device=x.device)
     _check_buffer(normed, (m, k), torch.bfloat16, x.device, "normed")
-    # A weight stored [K, N] (N-contiguous B) is copied K-contiguous first, as for dX.
+    # A weight stored [K, N] (N-contiguous B) is copied K-contiguous first (9216 x 2048, copy
+    # and product against direct: 16384 rows 478 / 496 us, 8192 rows 254 / 250, 4096 rows
+    # 155 / 146).
     b = k_contiguous_b(weight.T, m)
     _hip.call("ws_rmsnorm_gate_mm", x.data_ptr(), x.stride(0), norm_weight.data_ptr(),
               float(eps), rstd.data_ptr(), normed.data_ptr(), b.data_ptr(), b.stride(0),

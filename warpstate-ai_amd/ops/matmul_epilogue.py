@@ -72,7 +72,9 @@ def launch_swiglu_mm(a: torch.Tensor, b: torch.Tensor, algorithm: str = "tiled",
     tile_code = _hip.tile_code(block_m, 2 * block_n)
     if tile_code == 0:
         # A weight given as a row-major [K, 2H] B (N-contiguous) is copied K-contiguous
-        # first: the 256 x 256 paired kernel reads it 10-15 % faster that way.
+        # first. The paired kernel reads it 3-6 % faster that way, which pays for the copy
+        # from about 12000 rows on (11264 x 2048 weight, copy and product against direct:
+        # 16384 rows 587 / 611 us, 8192 rows 310 / 302, 4096 rows 163 / 150).
         from ops.fused_execution import k_contiguous_b
 
         b = k_contiguous_b(b, rows)
