@@ -52,3 +52,17 @@ def test_weight_is_copied_for_outputs_off_16_byte_pieces():
 def test_few_rows_never_pay_for_a_copy(rows):
     weight = torch.empty(65, 128, dtype=BF16)
     assert fx.gemm_b(_a("aligned", rows, 65), weight) is weight
+
+
+@pytest.mark.parametrize("rows,d,vocab,kind,stored,copied", [
+    (2048, 64, 1024, "aligned", False, True), (1023, 64, 1024, "aligned", False, False),
+    (2048, 64, 1027, "aligned", False, False), (2048, 64, 1028, "aligned", False, False),
+    (2048, 64, 1028, "aligned", True, True), (2048, 60, 1027, "aligned", False, True),
+    (2048, 64, 1027, "odd stride", False, True), (2048, 64, 1027, "odd address", False, True)])
+def test_head_weight_is_copied_where_a_kernel_reads_the_copy(rows, d, vocab, kind, stored, copied):
+    """A vocabulary off multiples of 8 with vector operands has padded chunk rows and no copy;
+    with any other operands the generic kernel takes it."""
+    weight = torch.empty(vocab, d, dtype=BF16)
+    copy = fx._head_weight_t(_a(kind, rows, d), weight, stored)
+    assert (copy is not None) == copied
+    assert copy is None or copy.shape == (d, vocab)

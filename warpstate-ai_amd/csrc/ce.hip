@@ -205,9 +205,9 @@ static int ce_chunk_dhidden(const CeChunk& c, const unsigned short* gl, const vo
                             long ld_out, const int* skip, hipStream_t s) {
   GemmParams q{};
   q.a = OperandDesc{gl, c.ldg, 1};
-  // B [vocab, d]: the head weight (d contiguous) or its transpose (vocab contiguous, whose
-  // rows are 16-byte pieces only for a vocabulary that is a multiple of 8).
-  q.b = weight_t && vocab % 8 == 0 ? OperandDesc{static_cast<const unsigned short*>(weight_t), vocab, 1}
+  // B [vocab, d]: the head weight (d contiguous) or its transpose (vocab contiguous), which has
+  // no 16-byte rows to go with padded chunk rows.
+  q.b = weight_t && c.ldg == vocab ? OperandDesc{static_cast<const unsigned short*>(weight_t), vocab, 1}
                  : OperandDesc{static_cast<const unsigned short*>(weight), 1, ld_weight};
   q.M = (int)c.r; q.N = (int)d; q.K = (int)vocab;
   q.skip_if = skip;

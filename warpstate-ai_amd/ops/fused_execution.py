@@ -471,12 +471,16 @@ def _check_state(state: CrossEntropyState, rows: int, vocab: int, device) -> Non
         raise ValueError("CrossEntropyState chunk_rows must lie in [1, rows]")
 
 
-def _head_weight_t(weight: torch.Tensor, rows: int) -> torch.Tensor | None:
+def _head_weight_t(hidden: torch.Tensor, weight: torch.Tensor, stored: bool = False
+                   ) -> torch.Tensor | None:
     """The head weight transposed for the dHidden GEMM (K-contiguous B) when there are enough
-    rows to amortize the copy, which has 16-byte rows only for a vocabulary that is a multiple
-    of 8."""
-    return (transpose(weight) if rows >= TRANSPOSE_MIN_ROWS and weight.shape[0] % 8 == 0
-            else None)
+    rows to amortize the copy. With a vocabulary that is no multiple of 8 the copy has no
+    16-byte rows: the vector GEMM over padded chunk rows then reads the weight as it is, and
+    only the generic kernel (operands that the vector loaders refuse, ``stored`` logits)
+    takes the copy."""
+    padded = (weight.shape[0] % 8 != 0 and not stored and _vector_rows(hidden)
+              and _vector_rows(weight))
+    return transpose(weight) if hidden.shape[0] >= TRANSPOSE_MIN_ROWS and not padded else None
 
 
 def linear_cross_entropy_forward(hidden: torch.Tensor, weight: torch.Tensor,
@@ -494,7 +498,7 @@ def linear_cross_entropy_forward(hidden: torch.Tensor, weight: torch.Tensor,
         if state.d != d:
             raise ValueError(f"The fused CrossEntropyState was built for d={state.d}, not {d}")
         workspace = state.backward_workspace(d)
-        weight_t = _head_weight_t(weight, rows)
+        weight_t = _head_weight_t(hidden, weight)
         # Kept for the backward's two-pass fallback (an upstream gradient that is not a
         # power of two).
         state.weight_t = weight_t
@@ -559,7 +563,7 @@ def linear_cross_entropy_backward(hidden: torch.Tensor, weight: torch.Tensor,
         return out
     workspace = state.backward_workspace(d)
     # The dHidden GEMM reads the head weight along the vocabulary: give it W^T rows.
-    weight_t = _head_weight_t(weight, rows)
+    weight_t = _head_weight_t(hidden, weight, state.logits is not None)
     _hip.call("ws_linear_ce_backward", hidden.data_ptr(), hidden.stride(0), weight.data_ptr(),
               weight.stride(0), None if weight_t is None else weight_t.data_ptr(),
               targets.data_ptr(), state.lse.data_ptr(), state.count.data_ptr(),
