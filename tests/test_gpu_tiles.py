@@ -95,13 +95,17 @@ def _run(epilogue, m, n, k, a_mn, b_n):
     return full
 
 
+# The gated projection's normalized operand is always row by row; a token-major A beside another
+# epilogue than the plain store runs on 256 x 256 tiles only.
+CASES = [(e, tile, a_mn) for e in (STORE, RESIDUAL, SIGMOID, SWIGLU, SWIGLU_BACKWARD)
+         for tile in TILES for a_mn in (0, 1)
+         if not a_mn or e == STORE or (tile == 0 and e != SIGMOID)]
+
+
 @pytest.mark.parametrize("b_n", [0, 1])
-@pytest.mark.parametrize("a_mn", [0, 1])
-@pytest.mark.parametrize("tile", list(TILES))
-@pytest.mark.parametrize("epilogue", [STORE, RESIDUAL, SIGMOID, SWIGLU, SWIGLU_BACKWARD])
+@pytest.mark.parametrize("epilogue,tile,a_mn", CASES)
 def test_products_are_exact(epilogue, tile, a_mn, b_n):
-    if epilogue == SIGMOID and a_mn:
-        pytest.skip("the normalized operand is written row by row")
+    ran = 0
     for k in SHORT + LONG:
         shape = gemm_shape(epilogue, a_mn, b_n, tile, k)
         if shape is None:
@@ -116,6 +120,10 @@ def test_products_are_exact(epilogue, tile, a_mn, b_n):
                   flush=True)
             full = _run(epilogue, rows, n, k, a_mn, b_n)
             assert (full[rows] == 7).all()
+            ran += 1
+    # There is no paired 64 x 64 tile, and none of these shapes is one for 128 x 128 alone under
+    # the SwiGLU backward.
+    assert ran or (epilogue, tile) in ((SWIGLU, 4), (SWIGLU_BACKWARD, 2))
 
 
 @pytest.mark.parametrize("store", [0, 1])
