@@ -278,7 +278,8 @@ int64_t ws_linear_ce_workspace_bytes(int64_t rows, int64_t vocab, int64_t d, int
  * the whole batch) go to the 256-byte aligned `workspace` and feed that chunk's dHidden
  * GEMM, split over the vocab with FP32 partials when the chunk alone would not fill the
  * GPU. `weight_t` (nullable) is the head weight transposed, [d, vocab] contiguous; when
- * given, the dHidden GEMM reads it instead of `weight`. `dweight` (nullable, FP32
+ * given, the dHidden GEMM reads it instead of `weight`, unless the vocabulary is no multiple
+ * of 8 and the vector kernels take the chunk. `dweight` (nullable, FP32
  * [vocab, d], row stride ld_dweight) receives the tied head weight's gradient, accumulated
  * per chunk as dweight += f32(r(G_chunk^T @ hidden_chunk)): the BF16 weight gradient of the
  * chunk's F.linear followed by FP32 accumulation (warpstate/model.py:321-331 under BF16

@@ -101,9 +101,8 @@ static inline int ce_dh_splits(long chunk, long d, long vocab) {
 // Row length of a chunk's logits and logit gradients: the vocabulary, or, when it is no
 // multiple of 8, the next multiple of 64, so that the chunk's GEMMs keep 16-byte rows and the
 // vector loaders (loss and gradients of 4352 x 1280 over 10883: 2265 us on the generic kernels,
-// 456 padded). The
-// padding holds zero gradients; the products read no weight row and write no gradient row
-// past the vocabulary.
+// 456 padded). The padding holds zero gradients; the products read no weight row and write no
+// gradient row past the vocabulary.
 static inline long ce_row(long vocab) { return vocab % 8 ? (vocab + 63) / 64 * 64 : vocab; }
 
 extern "C" int64_t ws_linear_ce_workspace_bytes(int64_t rows, int64_t vocab, int64_t d,
